@@ -213,3 +213,36 @@ def test_auto_fast_check_accepts_exactly_what_the_reasons_accept():
         residual_layer_norm(declined["x"], declined["branch"], declined["weight"],
                             declined["bias"])
     assert any("native hidden size must be one of" in str(w.message) for w in caught)
+
+
+@pytest.mark.parametrize("strides", [(640, 128, 1), (7, 128, 1)], ids=["dense", "free-size-1"])
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_outputs_follow_empty_like_and_are_written_whole(strides, deterministic):
+    """The outputs take the strides torch.empty_like gives (a dimension of size
+    1 keeps its own), and nothing in them depends on what the memory held:
+    deterministic mode, which would fill new tensors with NaN, and the default
+    mode over recycled NaN memory give the same bits."""
+    generator = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.empty_strided((1, 5, 128), strides, device="cuda").normal_(generator=generator)
+    branch = torch.empty_like(x).normal_(generator=generator)
+    weight, bias = torch.rand(2, 128, device="cuda", generator=generator)
+    assert x.is_contiguous() and x.stride() == strides
+    results = []
+    for fill in (float("nan"), 0.0):
+        dirty = [torch.full((5 * 128,), fill, device="cuda") for _ in range(12)]
+        del dirty
+        before = torch.are_deterministic_algorithms_enabled()
+        torch.use_deterministic_algorithms(deterministic)
+        try:
+            leaves = [t.detach().clone(memory_format=torch.preserve_format).requires_grad_()
+                      for t in (x, branch, weight, bias)]
+            outputs = residual_layer_norm(*leaves, 0.0, 1e-5, True, implementation="gfx950")
+            gradients = torch.autograd.grad(outputs, leaves,
+                                            [torch.ones_like(x), torch.cos(x)])
+        finally:
+            torch.use_deterministic_algorithms(before)
+        assert outputs[0].stride() == torch.empty_like(leaves[0]).stride()
+        assert outputs[1].stride() == torch.empty_like(leaves[0]).stride()
+        results.append([*outputs, *gradients])
+    for first, second in zip(*results):
+        assert torch.isfinite(first).all() and torch.equal(first, second)
