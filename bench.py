@@ -97,7 +97,7 @@ METRIC = "fwd & fwd+bwd achieved HBM GB/s (% of ~8 TB/s peak), rows/s at H=768"
 EPS = 1e-5
 TRAFFIC_FILE = REPO / "profiles" / "rln_backward_c1_traffic.json"
 CSRC = REPO / "gfx1010-kernels_amd" / "csrc"
-KERNEL_SOURCES = ("rln_device.h", "rln_api.hip", "rln_hidden.hip")
+KERNEL_SOURCES = ("rln_device.h", "rln_api.hip", "rln_hidden.hip", "rln_single.h", "rln_single.hip")
 PROBE_LIBRARY = REPO / "benchmarks" / "librln_probe_gfx950.so"
 # Back-to-back launches timed for the roofline kernel and the ceiling kernels.
 ROOFLINE_LAUNCHES = 400

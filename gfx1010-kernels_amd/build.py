@@ -53,6 +53,9 @@ HIP_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
+# The single-step kernels (every hidden size), one translation unit per pass.
+SINGLE_PASSES = (("forward", 1),)
+
 # One translation unit per row shape (every dtype and alignment variant of
 # its kernels), plus the C ABI; compiled in parallel, linked into one library.
 # Specialized hidden sizes, and the (slots per lane, waves per row) pairs of
@@ -94,6 +97,9 @@ def build_library(jobs: int | None = None, defines: tuple[str, ...] = (),
     build_dir.mkdir(parents=True, exist_ok=True)
     extra = [f"-D{define}" for define in defines]
     units = [(CSRC / "rln_api.hip", build_dir / "rln_api.o", extra)]
+    units += [(CSRC / "rln_single.hip", build_dir / f"rln_hidden_single_{name}.o",
+               [*extra, f"-DRLN_PASSES={passes}"])
+              for name, passes in SINGLE_PASSES]
     units += [
         (CSRC / "rln_hidden.hip", build_dir / f"rln_hidden_{hidden}.o",
          [*extra, f"-DRLN_HIDDEN={hidden}",

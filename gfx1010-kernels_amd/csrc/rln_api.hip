@@ -9,6 +9,7 @@
 #include <string>
 
 #include "rln_device.h"
+#include "rln_single.h"
 
 namespace rln {
 
@@ -334,6 +335,9 @@ int rln_forward(
         && aligned_to(updated, 16)
         && aligned_to(normalized, vector_alignment(normalized_dtype))
         && aligned_to(branch, vector_alignment(branch_dtype));
+    if (single_forward(rows, hidden, drop.active)) {
+        return launch_single_forward(a, hidden, branch_dtype, normalized_dtype, aligned);
+    }
     return with_shape<Pass::kForward>(hidden, rows, [&](auto shape) {
         return launch_forward_shape(a, shape, branch_dtype, normalized_dtype, aligned);
     });
