@@ -54,7 +54,7 @@ HIP_FLAGS = [
 ]
 
 # The single-step kernels (every hidden size), one translation unit per pass.
-SINGLE_PASSES = (("forward", 1),)
+SINGLE_PASSES = (("forward", 1), ("backward", 2))
 
 # One translation unit per row shape (every dtype and alignment variant of
 # its kernels), plus the C ABI; compiled in parallel, linked into one library.

@@ -89,20 +89,28 @@ struct SingleSplit {
 // so more waves share a row's Philox draws and loads ([341, 768] with
 // dropout 4.3 us on two waves of two slots, 4.8 on one of three; [512, 1024]
 // 4.8 against 5.8; [163, 1600] 4.0 against 4.4). Longer rows keep their order's
-// waves ([64, 4096] without dropout 4.3 us either way).
+// waves ([64, 4096] without dropout 4.3 us either way). The backward splits
+// rows of up to 768 columns finer, one slot per lane ([341, 768] 3.6 us on
+// three waves of one slot, 3.8 on one of three; [10923, 768] 28.2 against
+// 28.8), and keeps the order's waves above.
 template <Pass kPass>
 SingleSplit single_split(int64_t hidden, int64_t rows) {
     SingleSplit s{};
     s.order = sum_order<kPass>(hidden, rows);
-    if (hidden > 2048) {
+    const int64_t finest = kPass == Pass::kForward ? 2048 : 768;
+    if (hidden > finest) {
         s.path = SumPath::kDirect;
         s.vectors = s.order.vectors;
         s.parts = s.order.parts;
     } else {
-        s.vectors = hidden <= 256 ? 1 : 2;
+        s.vectors = kPass == Pass::kForward && hidden > 256 ? 2 : 1;
         const int64_t per_wave = 4 * kWaveSize * s.vectors;
         s.parts = static_cast<int>((hidden + per_wave - 1) / per_wave);
-        s.path = s.parts == 1 ? SumPath::kLanes : SumPath::kExchange;
+        // One wave of one slot holds the backward's row as its order does (at
+        // 128 columns the upper lanes add zeros).
+        s.path = s.parts > 1                ? SumPath::kExchange
+            : kPass == Pass::kForward ? SumPath::kLanes
+                                      : SumPath::kDirect;
     }
     s.groups = s.parts <= 2 ? 4 / s.parts : 1;
     s.reciprocal = (256 + s.parts - 1) / s.parts;
@@ -133,6 +141,76 @@ __device__ __forceinline__ void row_handoff(int parts) {
     } else {
         wave_handoff();
     }
+}
+
+// The backward runs single-step up to 12 M elements (2^24 above 6144 columns,
+// 2^23 for 256 and 4096-6144, 6 M for 1025-4095, 2^22 for 128), where the
+// walking backward's own costs - the fixed part of its row chains, and the
+// weight/bias atomics of its up to 256 blocks, which grow with the row length
+// and not with the rows - outweigh reading `updated` and grad_normalized a
+// second time. Measured (us, walking -> single-step), backward alone: [10, 768]
+// 4.2 -> 2.6, [682, 384] 5.8 -> 3.7, [163, 1600] 6.2 -> 3.8, [128, 4096] 9.3 ->
+// 4.8, [256, 8192] 35.0 -> 10.8, [4096, 512] 13.2 -> 9.6, [8192, 1024] 30.9 ->
+// 28.4, [12291, 384] fp32 20.6 -> 18.8, [2340, 7168] 71.0 -> 65.2; forward and
+// backward of the same batch, three or four batches in turn: [1024, 1024] 19.7
+// -> 12.3, [4096, 1024] 31.9 -> 28.4, [33111, 384] 77.8 -> 73.8, [2621, 1600]
+// 35.6 -> 32.9, [1024, 4096] 36.6 -> 30.2; and where the lines lie [32768, 128]
+// 32.1 -> 31.5, [61445, 128] fp16 out 47.2 -> 48.5, [32768, 256] 53.2 -> 50.6,
+// [52119, 256] fp32 branch 84.2 -> 85.0, [16555, 768] 77.4 -> 75.7, [21845, 768]
+// 95.8 -> 96.9, [3973, 1600] 45.0 -> 43.6, [2207, 2880] 45.2 -> 45.9, [2048,
+// 4096] 55.4 -> 55.4, [2048, 8192] 116.6 -> 110.9.
+//
+// Not where the walking backward runs its staggered twelve-wave blocks over
+// three row steps (768 columns, 7168 rows and more) with a 32-bit
+// grad_normalized: alone single-step is faster there too ([8192, 768] 24.2 ->
+// 21.6 us), but a forward right after it takes 1.9 us longer when the batches
+// that alternate fit the 256 MB Infinity Cache by half (forward + backward
+// over three batches 39.9 against 41.6 us, over eight 41.9 against 40.1; with
+// 16-bit gradients 39.2 -> 37.0 over three).
+inline bool single_backward(int64_t rows, int64_t hidden, int grad_normalized_dtype) {
+    const int64_t elements = rows * hidden;
+    if (grad_normalized_dtype == RLN_DTYPE_F32 && rows >= 7168
+        && backward_twelve_waves(hidden, rows)) {
+        return false;
+    }
+    const int64_t most = hidden == 128 ? 1 << 22
+        : hidden == 256               ? 1 << 23
+        : hidden <= 1024              ? 12 << 20
+        : hidden < 4096               ? 6 << 20
+        : hidden <= 6144              ? 1 << 23
+                                      : 1 << 24;
+    return elements <= most;
+}
+
+// Rows of one chunk: its blocks run on one XCD, and its slab blocks read again
+// from that XCD's L2 what its row blocks read. 64 rows (32 where a block has
+// three waves: whole steps of the slab blocks), fewer when there are fewer
+// rows than eight such chunks, one per XCD, so that every XCD has work.
+// Smaller chunks mean more weight/bias atomics, larger ones fall out of L2:
+// [8192, 768] 21.9 us at 32 rows, 22.7 at 64, 23.5 at 128; [8192, 1600] 44.5, 43.2,
+// 43.8; [16384, 128] 16.3, 10.4, 10.6.
+inline int64_t single_chunk_rows(int64_t rows, const SingleSplit& split) {
+    const int64_t most = split.waves() == 3 ? 32 : 64;
+    const int64_t spread = (rows + 7) / 8;
+    return spread < most ? (spread + 3) / 4 * 4 : most;
+}
+
+// Deterministic launches put one group of partials per chunk into a workspace
+// of backward_blocks(rows, hidden) groups, so a chunk may have to be larger.
+inline int64_t single_partial_rows(int64_t rows, int64_t hidden, const SingleSplit& split) {
+    const int64_t groups = backward_blocks(rows, hidden);
+    const int64_t least = (rows + groups - 1) / groups;
+    const int64_t chunk = single_chunk_rows(rows, split);
+    return least > chunk ? least : chunk;
+}
+
+// Past 64 rows per group of a full workspace, chunks fall out of L2 and the
+// walking backward is faster ([131072, 128] deterministic 57.5 against 64.8
+// us), and at 128 columns, where the row teams leave half their lanes idle
+// and nothing is gained on atomics, already from 4096 rows ([8192, 128] 9.1
+// against 11.1 us; [16384, 512] 30.7 -> 30.1 single-step).
+inline bool single_partials(int64_t rows, int64_t hidden) {
+    return rows <= (hidden == 128 ? 4096 : 64 * kBackwardMaxBlocks);
 }
 
 // `value` of the lanes of the wave's lower (upper) half in `low` (`high`), for
@@ -235,6 +313,62 @@ __device__ __forceinline__ float single_sum(const float (&slots)[V], float* shar
         const float sum_a = row_sum<kWaveSize>(partial_a);
         const float sum_b = row_sum<kWaveSize>(partial_b);
         return order.parts > 1 ? sum_a + sum_b : sum_a;
+    }
+}
+
+// The backward's two row sums at once, as single_sum: `shared` holds the pair
+// of every wave of the row (direct) or of every vector (exchange: one slot per
+// lane, one part in the order).
+template <int V, SumPath Path>
+__device__ __forceinline__ float2 single_pair_sum(const float (&q)[V], const float (&qx)[V],
+                                                  float2* shared, int parts, int part,
+                                                  const SumOrder& order) {
+    const int lane = threadIdx.x & (kWaveSize - 1);
+    if constexpr (Path == SumPath::kDirect) {
+        float2 partial = make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            partial.x += q[v];
+            partial.y += qx[v];
+        }
+        partial.x = row_sum<kWaveSize>(partial.x);
+        partial.y = row_sum<kWaveSize>(partial.y);
+        if (parts == 1) {
+            return partial;
+        }
+        if (lane == 0) {
+            shared[part] = partial;
+        }
+        __syncthreads();
+        float2 total = shared[0];
+#pragma unroll
+        for (int other = 1; other < kSingleMaxParts; ++other) {
+            const float2 next = shared[other];
+            total.x = other < parts ? total.x + next.x : total.x;
+            total.y = other < parts ? total.y + next.y : total.y;
+        }
+        return total;
+    } else {
+        static_assert(V == 1, "one slot per lane");
+        shared[part * kWaveSize + lane] = make_float2(q[0], qx[0]);
+        __syncthreads();
+        // Two or three slots of 64 lanes, or three of 32 (384 columns).
+        const float2* const first = shared + (lane & (order.lanes - 1));
+        const float2 a = first[0];
+        const float2 b = first[order.lanes];
+        const float2 c = first[order.vectors > 2 ? 2 * order.lanes : 0];
+        float2 partial = make_float2(a.x + b.x, a.y + b.y);
+        partial.x = order.vectors > 2 ? partial.x + c.x : partial.x;
+        partial.y = order.vectors > 2 ? partial.y + c.y : partial.y;
+        partial.x = row16_sum(partial.x);
+        partial.y = row16_sum(partial.y);
+        const float2 low =
+            make_float2(readlane_f32(partial.x, 0) + readlane_f32(partial.x, 16),
+                        readlane_f32(partial.y, 0) + readlane_f32(partial.y, 16));
+        const float2 high =
+            make_float2(readlane_f32(partial.x, 32) + readlane_f32(partial.x, 48),
+                        readlane_f32(partial.y, 32) + readlane_f32(partial.y, 48));
+        return order.lanes == kWaveSize ? make_float2(low.x + high.x, low.y + high.y) : low;
     }
 }
 
@@ -481,9 +615,246 @@ void rln_single_forward_kernel(SingleForwardArgs a) {
     }
 }
 
+struct SingleBackwardArgs {
+    const float* grad_updated;
+    const void* grad_normalized;
+    const float* updated;
+    const float* weight;
+    const float* mean;
+    const float* rstd;
+    const uint32_t* mask;
+    float* grad_x;
+    void* grad_branch;
+    float* grad_weight;
+    float* grad_bias;
+    float* partials;  // [chunks][2][hidden], or null for atomics
+    int64_t rows;
+    int hidden;
+    int parts;
+    int groups;
+    int reciprocal;
+    int row_blocks;   // per chunk
+    int chunk_rows;
+    int slab_waves;   // waves that share a slab's rows
+    int slabs;        // slabs of a slab block
+    float inv_hidden;
+    float scale;
+    int dropout;
+    SumOrder order;
+};
+
+constexpr int kSlabColumns = 64;
+constexpr int kSlabUnroll = 4;
+
+// Weight/bias sums of a chunk's rows over the slabs of 64 columns of one slab
+// block. They need no row sums (the forward saved mean and rstd), so they run
+// beside the chunk's row blocks instead of after them, read what those read
+// from the XCD's L2, and leave each block two sums per column to add: one add
+// per chunk and column instead of one per walking block, spread over the
+// kernel instead of at its end. A wave takes four rows of 16 lanes per step;
+// the order of the sums is fixed (steps, then the wave's four row slots, then
+// waves), so partials are reproducible bit for bit.
+template <typename GY, bool Aligned>
+__device__ __forceinline__ void single_slab(const SingleBackwardArgs& a, int block,
+                                            int64_t chunk, int64_t begin, int count) {
+    __shared__ float sums[kSingleMaxWaves][8][16];
+    const int lane = threadIdx.x & (kWaveSize - 1);
+    const int wave_in_block = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int waves = a.slab_waves;
+    const uint32_t hidden = a.hidden;
+    const int slab_in_block = wave_in_block >= waves ? 1 : 0;
+    const int wave = wave_in_block - slab_in_block * waves;
+    const int first_slab = block * a.slabs;
+    const uint32_t column =
+        (first_slab + slab_in_block) * kSlabColumns + (lane & 15) * 4;
+    // A slab past the row's end reads nothing and stores nothing.
+    const int64_t rows = column < hidden ? count : 0;
+    const int64_t extent = wave_uniform(rows) * hidden;
+    const rsrc_t u_in = input_range(a.updated, begin * hidden, extent);
+    const rsrc_t gy_in =
+        input_range(static_cast<const GY*>(a.grad_normalized), begin * hidden, extent);
+    const rsrc_t mean_in = input_range(a.mean, begin, count);
+    const rsrc_t rstd_in = input_range(a.rstd, begin, count);
+    const int sub = lane / 16;
+    const int steps = (count + 4 * waves - 1) / (4 * waves);
+    f32x4 acc_w = zero4();
+    f32x4 acc_b = zero4();
+    float means = 0.0f;
+    float rstds = 0.0f;
+    for (int step = 0; step < steps; step += kSlabUnroll) {
+        if (step % 16 == 0) {
+            // Lane i keeps the statistics of the wave's i-th row of 16 steps.
+            const uint32_t own = ((step + lane / 4) * waves + wave) * 4 + lane % 4;
+            means = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(mean_in, own * 4, 0, 0));
+            rstds = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(rstd_in, own * 4, 0, 0));
+        }
+        f32x4 u[kSlabUnroll];
+        typename Vector4<GY>::type gy[kSlabUnroll];
+#pragma unroll
+        for (int k = 0; k < kSlabUnroll; ++k) {
+            // Rows past the chunk's end read zeros: they add nothing.
+            const uint32_t row = ((step + k) * waves + wave) * 4 + sub;
+            u[k] = input4<float, Aligned, kSingleCachedLoad>(u_in, row * hidden + column);
+            gy[k] = input4<GY, Aligned, kSingleCachedLoad>(gy_in, row * hidden + column);
+        }
+#pragma unroll
+        for (int k = 0; k < kSlabUnroll; ++k) {
+            const int source = (step % 16 + k) * 4 + sub;
+            const float mean = __shfl(means, source);
+            const float rstd = __shfl(rstds, source);
+            const f32x4 g = widen4<GY>(gy[k]);
+            const f32x4 xhat = (u[k] - mean) * rstd;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc_w[e] = __builtin_fmaf(g[e], xhat[e], acc_w[e]);
+            }
+            acc_b = acc_b + g;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        acc_w[e] += __shfl_xor(acc_w[e], 16);
+        acc_w[e] += __shfl_xor(acc_w[e], 32);
+        acc_b[e] += __shfl_xor(acc_b[e], 16);
+        acc_b[e] += __shfl_xor(acc_b[e], 32);
+    }
+    if (lane < 16) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            sums[wave_in_block][e][lane] = acc_w[e];
+            sums[wave_in_block][4 + e][lane] = acc_b[e];
+        }
+    }
+    __syncthreads();
+    // Two waves per slab: its 64 weight sums and its 64 bias sums.
+    const int slab = threadIdx.x / (2 * kSlabColumns);
+    const int c = threadIdx.x % kSlabColumns;
+    const uint32_t out = (first_slab + slab) * kSlabColumns + c;
+    if (slab < a.slabs && out < hidden) {
+        const int which = (threadIdx.x / kSlabColumns) & 1;
+        float total = 0.0f;
+        for (int source = 0; source < waves; ++source) {
+            total += sums[slab * waves + source][4 * which + c % 4][c / 4];
+        }
+        if (a.partials != nullptr) {
+            a.partials[(chunk * 2 + which) * hidden + out] = total;
+        } else {
+            unsafeAtomicAdd((which ? a.grad_bias : a.grad_weight) + out, total);
+        }
+    }
+}
+
+// Input gradients: one row per team, as in the forward; weight/bias sums: slab
+// blocks of the same launch. gridDim.x = 8 * (row blocks + slab blocks of a
+// chunk) and consecutive blocks go to consecutive XCDs, so chunk 8 * y + x
+// runs on XCD x, its slab blocks behind its row blocks. (The placement is a
+// matter of speed alone.)
+template <int V, SumPath Path, typename B, typename GY, bool Aligned>
+__global__ __launch_bounds__(kSingleMaxWaves * kWaveSize)
+void rln_single_backward_kernel(SingleBackwardArgs a) {
+    const int local = blockIdx.x >> 3;
+    const int64_t chunk = static_cast<int64_t>(blockIdx.y) * 8 + (blockIdx.x & 7);
+    const int64_t begin = chunk * a.chunk_rows;
+    if (begin >= a.rows) {
+        return;
+    }
+    const int64_t left = a.rows - begin;
+    const int64_t end = begin + (left < a.chunk_rows ? left : a.chunk_rows);
+    if (local >= a.row_blocks) {
+        single_slab<GY, Aligned>(a, local - a.row_blocks, chunk, begin,
+                                 static_cast<int>(end - begin));
+        return;
+    }
+    // Direct: the wave totals of both sums; exchange: both of every vector of
+    // the block's rows (at most four waves).
+    constexpr int kShared = Path == SumPath::kExchange ? 4 * kWaveSize : kSingleMaxWaves;
+    __shared__ float2 shared[kShared];
+    const int lane = threadIdx.x & (kWaveSize - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int group = (wave * a.reciprocal) >> 8;
+    const int part = wave - group * a.parts;
+    const uint32_t hidden = a.hidden;
+    const int64_t team_row = begin + static_cast<int64_t>(local) * a.groups + group;
+    const bool valid = team_row < end;
+    const int64_t row = valid ? team_row : 0;
+    const int64_t count = valid ? hidden : 0;
+    const int64_t base = row * hidden;
+    // Absent inputs have empty descriptors: zeros, no memory access.
+    const bool has_gy = a.grad_normalized != nullptr;
+    const bool has_gu = a.grad_updated != nullptr;
+    const rsrc_t u_in = input_range(a.updated, base, count);
+    const rsrc_t gy_in = input_range(static_cast<const GY*>(a.grad_normalized),
+                                     has_gy ? base : 0, has_gy ? count : 0);
+    const rsrc_t gu_in = input_range(a.grad_updated, has_gu ? base : 0, has_gu ? count : 0);
+    const rsrc_t mask_in = input_range(a.mask, a.dropout ? row * (hidden / 32) : 0,
+                                       a.dropout ? count / 32 : 0);
+    const rsrc_t weight_in = input_range(a.weight, 0, hidden);
+    const float mean = a.mean[row];
+    const float rstd = a.rstd[row];
+    uint32_t column[V];
+    f32x4 u[V];
+    typename Vector4<GY>::type raw_gy[V];
+    f32x4 gu[V];
+    f32x4 w[V];
+    uint32_t bits[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        // What the slab blocks read again is loaded cached, the rest streams.
+        column[v] = ((v * a.parts + part) * kWaveSize + lane) * 4;
+        u[v] = input4<float, Aligned, kSingleCachedLoad>(u_in, column[v]);
+        raw_gy[v] = input4<GY, Aligned, kSingleCachedLoad>(gy_in, column[v]);
+        w[v] = input4<float, Aligned, kSingleCachedLoad>(weight_in, column[v]);
+        gu[v] = input4<float, Aligned, kSingleStreamLoad>(gu_in, column[v]);
+        bits[v] = __builtin_amdgcn_raw_buffer_load_b32(mask_in, column[v] / 32 * 4, 0,
+                                                       kSingleStreamLoad);
+    }
+    f32x4 gy[V];
+    f32x4 xhat[V];
+    float q_slots[V];
+    float qx_slots[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        gy[v] = widen4<GY>(raw_gy[v]);
+        xhat[v] = column[v] < hidden ? (u[v] - mean) * rstd : zero4();
+        const f32x4 q = gy[v] * w[v];
+        q_slots[v] = sum4(q);
+        qx_slots[v] =
+            (q.x * xhat[v].x + q.y * xhat[v].y) + (q.z * xhat[v].z + q.w * xhat[v].w);
+    }
+    const float2 totals = single_pair_sum<V, Path>(
+        q_slots, qx_slots, shared + group * a.parts * (Path == SumPath::kExchange ? kWaveSize : 1),
+        a.parts, part, a.order);
+    const float mean_q = totals.x * a.inv_hidden;
+    const float mean_qx = totals.y * a.inv_hidden;
+    const rsrc_t grad_x_out = output_range(a.grad_x, base, count);
+    const rsrc_t grad_branch_out = output_range(static_cast<B*>(a.grad_branch), base, count);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        f32x4 g = gu[v];
+        if (has_gy) {
+            const f32x4 q = gy[v] * w[v];
+            g = g + rstd * ((q - mean_q) - xhat[v] * mean_qx);
+        }
+        output4<Aligned>(grad_x_out, column[v] * 4, g, true);
+        if (a.dropout) {
+            const uint32_t nibble = bits[v] >> (column[v] % 32);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                g[e] = g[e] * (static_cast<float>((nibble >> e) & 1u) * a.scale);
+            }
+        }
+        output_convert4<B, Aligned>(grad_branch_out, column[v] * sizeof(B), g, true);
+    }
+}
+
 // Instantiated in rln_single.hip.
 int launch_single_forward(const ForwardArgs& a, int64_t hidden, int branch_dtype,
                           int normalized_dtype, bool aligned);
+// With kPartials, one group of partials per single_partial_rows rows.
+int launch_single_backward(const BackwardArgs& a, int64_t hidden, int branch_dtype,
+                           int grad_normalized_dtype, bool aligned);
 
 }  // namespace rln
 

@@ -6,6 +6,7 @@
 namespace rln {
 namespace {
 
+#if RLN_PASSES & 1
 // Calls `launch.template operator()<V, Path>()` for a forward split.
 template <typename Launch>
 int with_forward_split(const SingleSplit& split, Launch&& launch) {
@@ -19,6 +20,23 @@ int with_forward_split(const SingleSplit& split, Launch&& launch) {
     return split.vectors == 3 ? launch.template operator()<3, SumPath::kDirect>()
                               : launch.template operator()<4, SumPath::kDirect>();
 }
+#endif
+
+#if RLN_PASSES & 2
+// The same for a backward split.
+template <typename Launch>
+int with_backward_split(const SingleSplit& split, Launch&& launch) {
+    if (split.path == SumPath::kExchange) {
+        return launch.template operator()<1, SumPath::kExchange>();
+    }
+    switch (split.vectors) {
+        case 1: return launch.template operator()<1, SumPath::kDirect>();
+        case 2: return launch.template operator()<2, SumPath::kDirect>();
+        case 3: return launch.template operator()<3, SumPath::kDirect>();
+        default: return launch.template operator()<4, SumPath::kDirect>();
+    }
+}
+#endif
 
 }  // namespace
 
@@ -63,6 +81,61 @@ int launch_single_forward(const ForwardArgs& f, int64_t hidden, int branch_dtype
                         <<<grid, threads, 0, f.stream>>>(a);
                 }
                 return check_launch("rln_single_forward_kernel");
+            });
+        });
+    });
+}
+#endif
+
+#if RLN_PASSES & 2
+int launch_single_backward(const BackwardArgs& f, int64_t hidden, int branch_dtype,
+                           int grad_normalized_dtype, bool aligned) {
+    const SingleSplit split = single_split<Pass::kBackward>(hidden, f.rows);
+    SingleBackwardArgs a{};
+    a.grad_updated = f.grad_updated;
+    a.grad_normalized = f.grad_normalized;
+    a.updated = f.updated;
+    a.weight = f.weight;
+    a.mean = f.mean;
+    a.rstd = f.rstd;
+    a.mask = f.mask;
+    a.grad_x = f.grad_x;
+    a.grad_branch = f.grad_branch;
+    a.grad_weight = f.grad_weight;
+    a.grad_bias = f.grad_bias;
+    a.partials = (f.flags & kPartials) ? f.partials : nullptr;
+    a.rows = f.rows;
+    a.hidden = static_cast<int>(hidden);
+    a.parts = split.parts;
+    a.groups = split.groups;
+    a.reciprocal = split.reciprocal;
+    a.chunk_rows = static_cast<int>((f.flags & kPartials)
+        ? single_partial_rows(f.rows, hidden, split) : single_chunk_rows(f.rows, split));
+    a.row_blocks = (a.chunk_rows + split.groups - 1) / split.groups;
+    a.slabs = split.waves() >= 8 ? 2 : 1;
+    a.slab_waves = split.waves() / a.slabs;
+    a.inv_hidden = 1.0f / static_cast<float>(hidden);
+    a.scale = f.scale;
+    a.dropout = (f.flags & kDropout) ? 1 : 0;
+    a.order = split.order;
+    const int64_t slab_columns = static_cast<int64_t>(a.slabs) * kSlabColumns;
+    const int64_t slab_blocks =
+        (f.flags & kParameters) ? (hidden + slab_columns - 1) / slab_columns : 0;
+    const int64_t chunks = (f.rows + a.chunk_rows - 1) / a.chunk_rows;
+    const dim3 grid(static_cast<unsigned>(8 * (a.row_blocks + slab_blocks)),
+                    static_cast<unsigned>((chunks + 7) / 8));
+    const int threads = split.threads();
+    return with_dtype(branch_dtype, [&]<typename B>() {
+        return with_dtype(grad_normalized_dtype, [&]<typename GY>() {
+            return with_backward_split(split, [&]<int V, SumPath Path>() {
+                if (aligned) {
+                    rln_single_backward_kernel<V, Path, B, GY, true>
+                        <<<grid, threads, 0, f.stream>>>(a);
+                } else {
+                    rln_single_backward_kernel<V, Path, B, GY, false>
+                        <<<grid, threads, 0, f.stream>>>(a);
+                }
+                return check_launch("rln_single_backward_kernel");
             });
         });
     });

@@ -55,3 +55,94 @@ def test_small_rows(rows, hidden):
 @pytest.mark.parametrize("above", [0, 1])
 def test_forward_switch(hidden, rows, dropout_p, above):
     _run(rows + above, hidden, torch.float16, torch.float32, dropout_p)
+
+
+# The backward's last single-step row count and the first walked one.
+@pytest.mark.parametrize("hidden,rows", [(128, (1 << 22) // 128), (256, (1 << 23) // 256),
+                                         (768, (12 << 20) // 768), (1088, (6 << 20) // 1088),
+                                         (4096, (1 << 23) // 4096), (6208, (1 << 24) // 6208),
+                                         # the staggered walking backward among them
+                                         (768, 7679), (768, 7680), (768, 9216)])
+@pytest.mark.parametrize("above", [0, 1])
+def test_backward_switch(hidden, rows, above):
+    _run(rows + above, hidden, torch.float16, torch.bfloat16, 0.1)
+
+
+def _row_outputs(rows, hidden, inputs, grads, branch_dtype, dropout_p, deterministic=False):
+    """Forward and backward over the first `rows` rows, without weight/bias sums."""
+    from test_gpu_schedules import run
+
+    out = run((inputs[0], inputs[1], inputs[2], inputs[3], *grads), rows, torch.float32,
+              dropout_p, deterministic)
+    return {name: out[name] for name in ("updated", "normalized", "mean", "rstd", "mask", "grad_x",
+                                         "grad_branch")}, out["parameters"]
+
+
+@pytest.mark.parametrize("hidden", [128, 192, 256, 320, 384, 512, 576, 768, 832, 1024, 1088, 1600,
+                                    2048, 2112, 2880, 4096, 4160, 7168, 8192])
+@pytest.mark.parametrize("dropout_p", [0.0, 0.1])
+def test_single_step_rows_equal_walked_rows(hidden, dropout_p):
+    """A row's outputs are the same bits from the single-step kernels (a few
+    rows) and from the walking ones (enough rows to be above both rules; rows
+    of 768 and 6657-8192 columns stay below the sizes that change the walking
+    backward's own sums)."""
+    many = (1 << 24) // hidden + 3
+    inputs, grads = device_inputs(many, hidden, torch.bfloat16, seed=hidden)
+    print(f"[single step] rows {many} against 77 H={hidden} p={dropout_p}", flush=True)
+    walked, _ = _row_outputs(many, hidden, inputs, grads, torch.bfloat16, dropout_p)
+    single, _ = _row_outputs(77, hidden, inputs, grads, torch.bfloat16, dropout_p)
+    for name, value in single.items():
+        if name == "mask":
+            count = value.numel() if dropout_p else 0
+            assert torch.equal(value[:count], walked[name][:count])
+        else:
+            integer = {4: torch.int32, 2: torch.int16}[value.element_size()]
+            assert torch.equal(value.view(integer), walked[name][:77].view(integer)), name
+
+
+@pytest.mark.parametrize("rows,hidden", [(3, 384), (300, 192), (4096, 128), (4097, 128),
+                                         (9000, 256), (16384, 512), (16385, 512), (500, 2880),
+                                         (33, 8192)])
+def test_deterministic_partials(rows, hidden):
+    """Fixed-order weight/bias sums of single-step launches: chunks of few and
+    many rows, and the row counts that hand over to the walking backward. Bit
+    for bit the same twice, at the parity bar against float64."""
+    from test_gpu_schedules import check_parameter_sums, run
+
+    print(f"[single step] deterministic rows={rows} H={hidden}", flush=True)
+    inputs, grads = device_inputs(rows, hidden, torch.float16, seed=rows + hidden)
+    case = (*inputs, *grads)
+    first = run(case, rows, torch.float32, 0.1, True)
+    second = run(case, rows, torch.float32, 0.1, True)
+    assert torch.equal(first["parameters"], second["parameters"])
+    check_parameter_sums(first, grads[1], rows)
+
+
+@pytest.mark.parametrize("over", ["grad_normalized", "updated"])
+@pytest.mark.parametrize("rows,hidden", [(100, 768), (40, 2880)])
+def test_gradients_written_over_their_inputs(rows, hidden, over):
+    """grad_x in the memory of grad_normalized or `updated`: the same results
+    as in memory of its own."""
+    from gfx1010_kernels import _cabi
+
+    inputs, grads = device_inputs(rows, hidden, torch.float32, seed=rows)
+    updated, _, mean, rstd, mask = _C.residual_layer_norm_forward(*inputs, 0.1, EPS, True, 128)
+    print(f"[single step] grad_x over {over} rows={rows} H={hidden}", flush=True)
+    results = []
+    for in_place in (False, True):
+        saved = dict(grad_normalized=grads[1].clone(), updated=updated.clone())
+        grad_x = saved[over] if in_place else torch.empty_like(updated)
+        grad_branch = torch.empty_like(updated)
+        sums = torch.zeros(2, hidden, device="cuda")
+        _cabi.backward(
+            grads[0].data_ptr(), saved["grad_normalized"].data_ptr(), saved["updated"].data_ptr(),
+            inputs[2].data_ptr(), mean.data_ptr(), rstd.data_ptr(), mask.data_ptr(),
+            grad_x.data_ptr(), grad_branch.data_ptr(), _cabi.RLN_DTYPE_F32, sums[0].data_ptr(),
+            sums[1].data_ptr(), rows, hidden, 0.1, True, False, None, 0,
+            torch.cuda.current_stream().cuda_stream, accumulate_parameters=True)
+        torch.cuda.synchronize()
+        results.append((grad_x, grad_branch, sums))
+    assert torch.equal(results[0][0], results[1][0])
+    assert torch.equal(results[0][1], results[1][1])
+    # Two fp32 orders of sums over at most 100 values of order one.
+    assert torch.allclose(results[0][2], results[1][2], rtol=1e-5, atol=1e-4)
