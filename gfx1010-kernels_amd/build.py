@@ -53,8 +53,10 @@ HIP_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-# The single-step kernels (every hidden size), one translation unit per pass.
+# The single-step kernels (every hidden size), one translation unit per pass;
+# their first 14 argument words arrive in scalar registers (rln_single.h).
 SINGLE_PASSES = (("forward", 1), ("backward", 2))
+SINGLE_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
 
 # One translation unit per row shape (every dtype and alignment variant of
 # its kernels), plus the C ABI; compiled in parallel, linked into one library.
@@ -98,7 +100,7 @@ def build_library(jobs: int | None = None, defines: tuple[str, ...] = (),
     extra = [f"-D{define}" for define in defines]
     units = [(CSRC / "rln_api.hip", build_dir / "rln_api.o", extra)]
     units += [(CSRC / "rln_single.hip", build_dir / f"rln_hidden_single_{name}.o",
-               [*extra, f"-DRLN_PASSES={passes}"])
+               [*extra, *SINGLE_FLAGS, f"-DRLN_PASSES={passes}"])
               for name, passes in SINGLE_PASSES]
     units += [
         (CSRC / "rln_hidden.hip", build_dir / f"rln_hidden_{hidden}.o",

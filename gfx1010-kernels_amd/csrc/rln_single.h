@@ -411,37 +411,70 @@ __device__ __forceinline__ typename Vector4<T>::type input4(rsrc_t r, uint32_t i
     }
 }
 
+// What a kernel needs to issue its first loads comes as arguments of its own,
+// at most 14 words, which the build has the hardware preload into scalar
+// registers at wave launch (-amdgpu-kernarg-preload-count); the rest follows in
+// a struct. Scalar loads return out of order, so the first use of one waits
+// for every one issued: with all arguments in one struct the first row load
+// waited for several cold lines of arguments. Measured (us, one struct ->
+// separate words -> preloaded): forward [8, 768] bf16 2.92 -> 2.89 -> 2.79,
+// [1024, 384] with dropout 4.29 -> 4.18 -> 4.06, [2048, 768] with dropout 6.67
+// -> 6.70 -> 6.24; backward [1024, 384] 3.96 -> 3.98 -> 3.75, [64, 1600] 3.31 ->
+// 3.33 -> 3.21.
+struct SplitWord {
+    uint32_t bits;
+    static SplitWord of(const SingleSplit& s) {
+        return {static_cast<uint32_t>(s.parts | s.groups << 4 | s.reciprocal << 8
+                                      | s.order.parts << 18 | s.order.vectors << 22
+                                      | (s.order.lanes / 16) << 25)};
+    }
+    __device__ __forceinline__ int parts() const { return bits & 15; }
+    __device__ __forceinline__ int groups() const { return (bits >> 4) & 15; }
+    __device__ __forceinline__ int reciprocal() const { return (bits >> 8) & 1023; }
+    __device__ __forceinline__ SumOrder order() const {
+        return {static_cast<int>(bits >> 25) * 16, static_cast<int>((bits >> 22) & 7),
+                static_cast<int>((bits >> 18) & 15)};
+    }
+};
+
+// Dropout of a single-step forward: off, or the stream's launch width (0: the
+// library's layout) and whether the seed is a device pointer.
+struct DropWord {
+    uint32_t bits;
+    static DropWord of(int dropout, const PhiloxArgs& philox) {
+        return {static_cast<uint32_t>((dropout ? 1 : 0) | (philox.seed_ptr ? 2 : 0)
+                                      | philox.threads << 2)};
+    }
+    __device__ __forceinline__ bool on() const { return bits & 1; }
+    __device__ __forceinline__ bool captured() const { return bits & 2; }
+    __device__ __forceinline__ int threads() const { return bits >> 2; }
+};
+
 struct SingleForwardArgs {
-    const float* x;
-    const void* branch;
+    uint32_t threshold;
+    float scale;
     const float* weight;
     const float* bias;
     float* updated;
     void* normalized;
+    uint32_t* mask;
     float* mean;
     float* rstd;
-    uint32_t* mask;
-    float* zero_weight;
-    float* zero_bias;
-    int64_t rows;
-    int hidden;
-    int parts;
-    int groups;
-    int reciprocal;
     float inv_hidden;  // 1.0f / hidden, rounded once on the host
     float eps;
-    int dropout;
-    float scale;
-    uint32_t threshold;
-    SumOrder order;
-    PhiloxArgs philox;
+    float* zero_weight;
+    float* zero_bias;
 };
 
 // One row per team of `parts` waves; slot v of lane l of part p holds columns
 // 4 * ((v * parts + p) * 64 + l) .. + 3.
 template <int V, SumPath Path, typename B, typename N, bool Aligned>
 __global__ __launch_bounds__(kSingleMaxWaves * kWaveSize)
-void rln_single_forward_kernel(SingleForwardArgs a) {
+void rln_single_forward_kernel(const float* x_rows, const B* branch_rows, int rows, uint32_t hidden,
+                               SplitWord split, DropWord drop,
+                               const int64_t* __restrict__ seed_or_value, uint64_t philox_offset,
+                               const int64_t* __restrict__ offset_ptr,
+                               SingleForwardArgs a) {
     // [0] the mean's sum, [1] the variance's: one float per wave of the row
     // (direct), or one per vector of the block's rows (exchange, at most four
     // waves).
@@ -452,28 +485,30 @@ void rln_single_forward_kernel(SingleForwardArgs a) {
     __shared__ uint64_t keep[4][16];
     const int lane = threadIdx.x & (kWaveSize - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-    const int group = (wave * a.reciprocal) >> 8;
-    const int part = wave - group * a.parts;
-    const uint32_t hidden = a.hidden;
+    const int parts = split.parts();
+    const SumOrder order = split.order();
+    const int group = (wave * split.reciprocal()) >> 8;
+    const int part = wave - group * parts;
     // A team past the last row reads and writes nothing (empty descriptors),
     // but meets its block's barriers.
-    const int64_t team_row = static_cast<int64_t>(blockIdx.x) * a.groups + group;
-    const bool valid = team_row < a.rows;
+    const int team_row = blockIdx.x * split.groups() + group;
+    const bool valid = team_row < rows;
     const int64_t row = valid ? team_row : 0;
     const int64_t count = valid ? hidden : 0;
     const int64_t base = row * hidden;
-    const int row_shared = Path == SumPath::kExchange ? group * V * a.parts * kWaveSize : 0;
+    const int row_shared = Path == SumPath::kExchange ? group * V * parts * kWaveSize : 0;
 
     // The Philox key and position first: the draws hang on them, and under
     // graph capture they come from memory.
     uint32_t key0 = 0;
     uint32_t key1 = 0;
     uint64_t position = 0;
-    if (a.dropout) {
-        const uint64_t seed = a.philox.seed_ptr ? static_cast<uint64_t>(*a.philox.seed_ptr)
-                                                : a.philox.seed;
-        const uint64_t offset = a.philox.offset
-            + (a.philox.offset_ptr ? static_cast<uint64_t>(*a.philox.offset_ptr) : 0);
+    const bool dropout = drop.on();
+    if (dropout) {
+        const uint64_t seed = drop.captured() ? static_cast<uint64_t>(*seed_or_value)
+                                              : reinterpret_cast<uint64_t>(seed_or_value);
+        const uint64_t offset =
+            philox_offset + (offset_ptr ? static_cast<uint64_t>(*offset_ptr) : 0);
         key0 = static_cast<uint32_t>(seed);
         key1 = static_cast<uint32_t>(seed >> 32);
         position = offset / 4;
@@ -483,11 +518,11 @@ void rln_single_forward_kernel(SingleForwardArgs a) {
     typename Vector4<B>::type branch[V];
     f32x4 w[V];
     f32x4 b[V];
-    const rsrc_t x_in = input_range(a.x, base, count);
-    const rsrc_t branch_in = input_range(static_cast<const B*>(a.branch), base, count);
+    const rsrc_t x_in = input_range(x_rows, base, count);
+    const rsrc_t branch_in = input_range(branch_rows, base, count);
 #pragma unroll
     for (int v = 0; v < V; ++v) {
-        column[v] = ((v * a.parts + part) * kWaveSize + lane) * 4;
+        column[v] = ((v * parts + part) * kWaveSize + lane) * 4;
         x[v] = input4<float, Aligned, kSingleStreamLoad>(x_in, column[v]);
         branch[v] = input4<B, Aligned, kSingleStreamLoad>(branch_in, column[v]);
     }
@@ -510,17 +545,17 @@ void rln_single_forward_kernel(SingleForwardArgs a) {
     // Keep bits of each slot in bits 0-3 of `bits`; both layouts of the
     // stream are those of the walking forward (rln_device.h).
     uint32_t bits[V];
-    if (a.dropout && a.philox.threads != 0) {
+    if (dropout && drop.threads() != 0) {
         // The reference's stream: thread t of the row draws `calls` Philox
         // blocks, value `item` of which decides column t + item * threads.
         // 64 consecutive threads and one call are a unit; a ballot over value
         // e of a unit covers 64 consecutive columns, two words of the mask.
-        const int threads = a.philox.threads;
+        const int threads = drop.threads();
         const int per_item = threads / kWaveSize;
-        const int items = (a.hidden + threads - 1) / threads;
+        const int items = (static_cast<int>(hidden) + threads - 1) / threads;
         const int calls = (items + 3) / 4;  // 1 or 2
-        const int chunks = a.hidden / kWaveSize;
-        for (int unit = part; unit < per_item * calls; unit += a.parts) {
+        const int chunks = hidden / kWaveSize;
+        for (int unit = part; unit < per_item * calls; unit += parts) {
             const int k = calls == 2 ? unit >> 1 : unit;
             const int n = calls == 2 ? unit & 1 : 0;
             const uint64_t low = position + n;
@@ -541,17 +576,17 @@ void rln_single_forward_kernel(SingleForwardArgs a) {
                 }
             }
         }
-        row_handoff(a.parts);
+        row_handoff(parts);
         const uint32_t* const words = reinterpret_cast<const uint32_t*>(keep[group]);
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             bits[v] = column[v] < hidden ? words[column[v] / 32] >> (column[v] % 32) : 0u;
         }
-        if (part == 0 && lane < a.hidden / 32) {
+        if (part == 0 && lane < static_cast<int>(hidden / 32)) {
             output_b32(output_range(a.mask, row * (hidden / 32), count / 32), lane * 4,
                        words[lane], true);
         }
-    } else if (a.dropout) {
+    } else if (dropout) {
         const rsrc_t mask_out = output_range(a.mask, row * (hidden / 32), count / 32);
 #pragma unroll
         for (int v = 0; v < V; ++v) {
@@ -576,7 +611,7 @@ void rln_single_forward_kernel(SingleForwardArgs a) {
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         f32x4 d = widen4<B>(branch[v]);
-        if (a.dropout) {
+        if (dropout) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 d[e] = round_to_branch<B>(d[e] * static_cast<float>((bits[v] >> e) & 1u)
@@ -587,15 +622,15 @@ void rln_single_forward_kernel(SingleForwardArgs a) {
         output4<Aligned>(updated_out, column[v] * 4, u[v], true);
         slots[v] = sum4(u[v]);  // lanes past the row hold zeros
     }
-    const float mean = single_sum<V, Path>(slots, &shared[0][row_shared], a.parts, part,
-                                             a.order) * a.inv_hidden;
+    const float mean = single_sum<V, Path>(slots, &shared[0][row_shared], parts, part,
+                                             order) * a.inv_hidden;
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         u[v] = column[v] < hidden ? u[v] - mean : zero4();
         slots[v] = (u[v].x * u[v].x + u[v].y * u[v].y) + (u[v].z * u[v].z + u[v].w * u[v].w);
     }
-    const float variance = single_sum<V, Path>(slots, &shared[1][row_shared], a.parts, part,
-                                                 a.order) * a.inv_hidden;
+    const float variance = single_sum<V, Path>(slots, &shared[1][row_shared], parts, part,
+                                                 order) * a.inv_hidden;
     const float rstd = rsqrtf(variance + a.eps);
     if (part == 0 && lane == 0) {
         output_b32(output_range(a.mean, row, valid ? 1 : 0), 0,
@@ -616,31 +651,20 @@ void rln_single_forward_kernel(SingleForwardArgs a) {
 }
 
 struct SingleBackwardArgs {
+    int row_blocks;  // per chunk
+    int slab_waves;  // waves that share a slab's rows
+    int slabs;       // slabs of a slab block
+    int dropout;
     const float* grad_updated;
-    const void* grad_normalized;
-    const float* updated;
-    const float* weight;
-    const float* mean;
-    const float* rstd;
     const uint32_t* mask;
+    const float* weight;
     float* grad_x;
     void* grad_branch;
+    float inv_hidden;
+    float scale;
     float* grad_weight;
     float* grad_bias;
     float* partials;  // [chunks][2][hidden], or null for atomics
-    int64_t rows;
-    int hidden;
-    int parts;
-    int groups;
-    int reciprocal;
-    int row_blocks;   // per chunk
-    int chunk_rows;
-    int slab_waves;   // waves that share a slab's rows
-    int slabs;        // slabs of a slab block
-    float inv_hidden;
-    float scale;
-    int dropout;
-    SumOrder order;
 };
 
 constexpr int kSlabColumns = 64;
@@ -655,13 +679,14 @@ constexpr int kSlabUnroll = 4;
 // the order of the sums is fixed (steps, then the wave's four row slots, then
 // waves), so partials are reproducible bit for bit.
 template <typename GY, bool Aligned>
-__device__ __forceinline__ void single_slab(const SingleBackwardArgs& a, int block,
+__device__ __forceinline__ void single_slab(const SingleBackwardArgs& a, const float* updated,
+                                            const GY* grad_normalized, const float* means_in,
+                                            const float* rstds_in, uint32_t hidden, int block,
                                             int64_t chunk, int64_t begin, int count) {
     __shared__ float sums[kSingleMaxWaves][8][16];
     const int lane = threadIdx.x & (kWaveSize - 1);
     const int wave_in_block = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int waves = a.slab_waves;
-    const uint32_t hidden = a.hidden;
     const int slab_in_block = wave_in_block >= waves ? 1 : 0;
     const int wave = wave_in_block - slab_in_block * waves;
     const int first_slab = block * a.slabs;
@@ -670,11 +695,11 @@ __device__ __forceinline__ void single_slab(const SingleBackwardArgs& a, int blo
     // A slab past the row's end reads nothing and stores nothing.
     const int64_t rows = column < hidden ? count : 0;
     const int64_t extent = wave_uniform(rows) * hidden;
-    const rsrc_t u_in = input_range(a.updated, begin * hidden, extent);
+    const rsrc_t u_in = input_range(updated, begin * hidden, extent);
     const rsrc_t gy_in =
-        input_range(static_cast<const GY*>(a.grad_normalized), begin * hidden, extent);
-    const rsrc_t mean_in = input_range(a.mean, begin, count);
-    const rsrc_t rstd_in = input_range(a.rstd, begin, count);
+        input_range(grad_normalized, begin * hidden, extent);
+    const rsrc_t mean_in = input_range(means_in, begin, count);
+    const rsrc_t rstd_in = input_range(rstds_in, begin, count);
     const int sub = lane / 16;
     const int steps = (count + 4 * waves - 1) / (4 * waves);
     f32x4 acc_w = zero4();
@@ -753,17 +778,21 @@ __device__ __forceinline__ void single_slab(const SingleBackwardArgs& a, int blo
 // matter of speed alone.)
 template <int V, SumPath Path, typename B, typename GY, bool Aligned>
 __global__ __launch_bounds__(kSingleMaxWaves * kWaveSize)
-void rln_single_backward_kernel(SingleBackwardArgs a) {
+void rln_single_backward_kernel(const float* updated, const GY* grad_normalized,
+                                const float* means, const float* rstds, int rows,
+                                uint32_t hidden, SplitWord split, int chunk_rows,
+                                SingleBackwardArgs a) {
     const int local = blockIdx.x >> 3;
     const int64_t chunk = static_cast<int64_t>(blockIdx.y) * 8 + (blockIdx.x & 7);
-    const int64_t begin = chunk * a.chunk_rows;
-    if (begin >= a.rows) {
+    const int64_t begin = chunk * chunk_rows;
+    if (begin >= rows) {
         return;
     }
-    const int64_t left = a.rows - begin;
-    const int64_t end = begin + (left < a.chunk_rows ? left : a.chunk_rows);
+    const int64_t left = rows - begin;
+    const int64_t end = begin + (left < chunk_rows ? left : chunk_rows);
     if (local >= a.row_blocks) {
-        single_slab<GY, Aligned>(a, local - a.row_blocks, chunk, begin,
+        single_slab<GY, Aligned>(a, updated, grad_normalized, means, rstds, hidden,
+                                 local - a.row_blocks, chunk, begin,
                                  static_cast<int>(end - begin));
         return;
     }
@@ -773,26 +802,25 @@ void rln_single_backward_kernel(SingleBackwardArgs a) {
     __shared__ float2 shared[kShared];
     const int lane = threadIdx.x & (kWaveSize - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-    const int group = (wave * a.reciprocal) >> 8;
-    const int part = wave - group * a.parts;
-    const uint32_t hidden = a.hidden;
-    const int64_t team_row = begin + static_cast<int64_t>(local) * a.groups + group;
+    const int parts = split.parts();
+    const int group = (wave * split.reciprocal()) >> 8;
+    const int part = wave - group * parts;
+    const int64_t team_row = begin + static_cast<int64_t>(local) * split.groups() + group;
     const bool valid = team_row < end;
     const int64_t row = valid ? team_row : 0;
     const int64_t count = valid ? hidden : 0;
     const int64_t base = row * hidden;
     // Absent inputs have empty descriptors: zeros, no memory access.
-    const bool has_gy = a.grad_normalized != nullptr;
+    const bool has_gy = grad_normalized != nullptr;
     const bool has_gu = a.grad_updated != nullptr;
-    const rsrc_t u_in = input_range(a.updated, base, count);
-    const rsrc_t gy_in = input_range(static_cast<const GY*>(a.grad_normalized),
-                                     has_gy ? base : 0, has_gy ? count : 0);
+    const rsrc_t u_in = input_range(updated, base, count);
+    const rsrc_t gy_in = input_range(grad_normalized, has_gy ? base : 0, has_gy ? count : 0);
     const rsrc_t gu_in = input_range(a.grad_updated, has_gu ? base : 0, has_gu ? count : 0);
     const rsrc_t mask_in = input_range(a.mask, a.dropout ? row * (hidden / 32) : 0,
                                        a.dropout ? count / 32 : 0);
     const rsrc_t weight_in = input_range(a.weight, 0, hidden);
-    const float mean = a.mean[row];
-    const float rstd = a.rstd[row];
+    const float mean = means[row];
+    const float rstd = rstds[row];
     uint32_t column[V];
     f32x4 u[V];
     typename Vector4<GY>::type raw_gy[V];
@@ -802,7 +830,7 @@ void rln_single_backward_kernel(SingleBackwardArgs a) {
 #pragma unroll
     for (int v = 0; v < V; ++v) {
         // What the slab blocks read again is loaded cached, the rest streams.
-        column[v] = ((v * a.parts + part) * kWaveSize + lane) * 4;
+        column[v] = ((v * parts + part) * kWaveSize + lane) * 4;
         u[v] = input4<float, Aligned, kSingleCachedLoad>(u_in, column[v]);
         raw_gy[v] = input4<GY, Aligned, kSingleCachedLoad>(gy_in, column[v]);
         w[v] = input4<float, Aligned, kSingleCachedLoad>(weight_in, column[v]);
@@ -824,8 +852,8 @@ void rln_single_backward_kernel(SingleBackwardArgs a) {
             (q.x * xhat[v].x + q.y * xhat[v].y) + (q.z * xhat[v].z + q.w * xhat[v].w);
     }
     const float2 totals = single_pair_sum<V, Path>(
-        q_slots, qx_slots, shared + group * a.parts * (Path == SumPath::kExchange ? kWaveSize : 1),
-        a.parts, part, a.order);
+        q_slots, qx_slots, shared + group * parts * (Path == SumPath::kExchange ? kWaveSize : 1),
+        parts, part, split.order());
     const float mean_q = totals.x * a.inv_hidden;
     const float mean_qx = totals.y * a.inv_hidden;
     const rsrc_t grad_x_out = output_range(a.grad_x, base, count);
