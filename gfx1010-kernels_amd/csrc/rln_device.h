@@ -172,11 +172,11 @@
 // nt = 2, sc1 = 16. Launches over fewer than RLN_WRITE_THROUGH_ELEMENTS
 // elements write through the caches at system scope (sc0 | sc1), so that no
 // dirty line is left in L2 for the end-of-kernel release to write back;
-// larger launches store non-temporally. Measured on MI355X (bench.py --ab,
-// alternated): C1 [8192, 768] step 39.1 us write-through against 40.3 us
-// non-temporal (forward 14.8 against 17.0 us); at 2^26+ elements
-// non-temporal wins by 1-7 % (C3 358.7 against 371.6 us, [262144, 384]
-// 541 against 555 us), and so at [8192, 1600] (83.3 against 85.7 us). The
+// larger launches store non-temporally (the forward from the larger sizes
+// below). Measured on MI355X (bench.py --ab, alternated): C1 [8192, 768] step
+// 39.1 us write-through against 40.3 us non-temporal (forward 14.8 against
+// 17.0 us); at 2^26+ elements both passes write-through lose 1-7 % (C3 358.7
+// against 371.6 us, [262144, 384] 541 against 555 us). The
 // streaming probe at C1 (benchmarks/rln_probe.hip): forward-shaped pass 15.2
 // us write-through against 15.8 us plain and 18.8 us non-temporal.
 #ifndef RLN_SMALL_STORE_POLICY
@@ -188,8 +188,20 @@
 #ifndef RLN_WRITE_THROUGH_ELEMENTS
 #define RLN_WRITE_THROUGH_ELEMENTS (1ll << 23)
 #endif
+// The forward writes through up to larger launches: 2^24 elements, 2^25 for
+// rows of 512 columns and more, 2^26 for 1024 and more. Its outputs are then in the Infinity Cache, not
+// in L2 lines still to be written back, when the kernel ends: it ends sooner and
+// a backward that follows reads them faster. Measured (us, non-temporal ->
+// write-through): forward without dropout [6001, 2880] bf16 40.5 -> 38.7,
+// [32768, 1024] 81.3 -> 75.7, [8192, 4096] 85.2 -> 78.1; forward and backward
+// of the same batch [46340, 256] 69.6 -> 65.8, [43690, 768] 184.6 -> 178.1,
+// with dropout [17139, 768] +6.9 %, [8192, 1600] +5.4 %, [6427, 2048] +7.1 %,
+// [65536, 256] +2 to +4 %, [65536, 1024] +1.2 %, [16384, 4096] +1.5 %; and
+// past the lines [262144, 128] -1 %, [131072, 256] 0 %, [87381, 768] -0.8 %,
+// [174762, 768] -1.0 %, [131072, 1024] -0.6 to +0.3 %. (A large backward loses
+// 1-3 %.) The switch is the line of the shortest rows.
 #ifndef RLN_FWD_WRITE_THROUGH_ELEMENTS
-#define RLN_FWD_WRITE_THROUGH_ELEMENTS RLN_WRITE_THROUGH_ELEMENTS
+#define RLN_FWD_WRITE_THROUGH_ELEMENTS (1ll << 24)
 #endif
 #ifndef RLN_BWD_WRITE_THROUGH_ELEMENTS
 #define RLN_BWD_WRITE_THROUGH_ELEMENTS RLN_WRITE_THROUGH_ELEMENTS
@@ -845,7 +857,12 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // The descriptor's fourth word for a raw (untyped, unswizzled) buffer.
 constexpr int kRawBufferWord3 = 0x00020000;
-constexpr int64_t kForwardWriteThroughElements = RLN_FWD_WRITE_THROUGH_ELEMENTS;
+inline int forward_write_through(int64_t rows, int64_t hidden) {
+    const int64_t line = hidden >= 1024 ? 4 * RLN_FWD_WRITE_THROUGH_ELEMENTS
+        : hidden >= 512                 ? 2 * RLN_FWD_WRITE_THROUGH_ELEMENTS
+                                        : RLN_FWD_WRITE_THROUGH_ELEMENTS;
+    return rows * hidden <= line ? 1 : 0;
+}
 constexpr int64_t kBackwardWriteThroughElements = RLN_BWD_WRITE_THROUGH_ELEMENTS;
 
 // `value` of the wave's first active lane, in scalar registers.
@@ -2158,7 +2175,7 @@ int launch_forward_walk(const ForwardArgs& a, S shape) {
         a.threshold,
         a.philox,
         forward_paced(a.rows, shape.hidden()),
-        a.rows * shape.hidden() < kForwardWriteThroughElements ? 1 : 0);
+        forward_write_through(a.rows, shape.hidden()));
     return check_launch("rln_forward_kernel");
 }
 
