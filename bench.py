@@ -1506,6 +1506,30 @@ def kernel_name(kernel: str, workload: Workload) -> str:
             f"{types[workload.normalized]}, true{ring if forward else ''}>")
 
 
+def launched_kernel(kernel: str, workload: Workload) -> str:
+    """The kernel this workload launches: kernel_name()'s walking instance, or
+    the single-step kernel where the library's rules (rln_single.h
+    single_forward, single_backward, single_partials) take it."""
+    rows, hidden = workload.rows, workload.hidden
+    elements = rows * hidden
+    if kernel == "rln_forward_kernel":
+        if hidden > 4096 and not workload.dropout_p:
+            single = elements <= 1 << 17
+        else:
+            single = rows <= 6144 and elements <= (1 << 21 if hidden <= 1280 else 1 << 20)
+    else:
+        most = (1 << 22 if hidden == 128 else 1 << 23 if hidden == 256 else
+                12 << 20 if hidden <= 1024 else 6 << 20 if hidden < 4096 else
+                1 << 23 if hidden <= 6144 else 1 << 24)
+        single = elements <= most and not (
+            workload.normalized == "f32" and rows >= 7168 and backward_twelve_waves(hidden, rows))
+        if workload.deterministic:
+            single = single and rows <= (4096 if hidden == 128 else 64 * 256)
+    if not single:
+        return kernel_name(kernel, workload)
+    return f"rln::{kernel.replace('rln_', 'rln_single_')} ({workload.branch}, {workload.normalized})"
+
+
 def backward_twelve_waves(hidden: int, rows: int) -> bool:
     """Whether the backward runs twelve-wave blocks (rln_device.h
     backward_twelve_waves): 768 columns over 2048-9216 rows whose last row
@@ -1586,7 +1610,7 @@ def result_line(torch, workload: Workload, timing: dict, steps: int, warmup: int
         "algorithmic_bytes_per_step": total,
         "roofline": {
             "bound": "hbm",
-            "kernel": kernel_name(dominant, workload),
+            "kernel": launched_kernel(dominant, workload),
             "achieved": round(dominant_gbps, 2),
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",
