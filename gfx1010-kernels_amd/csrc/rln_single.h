@@ -213,6 +213,25 @@ inline bool single_partials(int64_t rows, int64_t hidden) {
     return rows <= (hidden == 128 ? 4096 : 64 * kBackwardMaxBlocks);
 }
 
+// A block's LDS array of row sums: its length, where the sums of the block's
+// row `group` begin, and how many elements from there its lanes read. Direct:
+// one per wave; the lanes read kSingleMaxParts of them in a fixed loop and drop
+// those past the row's waves, so the array reaches that far past the last row's
+// first. Exchange: one per vector of the block's rows (at most four waves).
+constexpr int single_shared_size(SumPath path, int vectors) {
+    return path == SumPath::kExchange ? vectors * 4 * kWaveSize
+                                      : kSingleMaxWaves + kSingleMaxParts;
+}
+constexpr int single_shared_first(SumPath path, int vectors, int parts, int group) {
+    return group * parts * (path == SumPath::kExchange ? vectors * kWaveSize : 1);
+}
+constexpr int single_shared_read(SumPath path, int parts, const SumOrder& order) {
+    if (path == SumPath::kExchange) {
+        return order.vectors * order.parts * order.lanes;
+    }
+    return parts > 1 ? kSingleMaxParts : 0;  // one wave keeps its sum in registers
+}
+
 // `value` of the lanes of the wave's lower (upper) half in `low` (`high`), for
 // the lanes of both halves.
 __device__ __forceinline__ void split_halves(float value, float& low, float& high) {
@@ -475,11 +494,8 @@ void rln_single_forward_kernel(const float* x_rows, const B* branch_rows, int ro
                                const int64_t* __restrict__ seed_or_value, uint64_t philox_offset,
                                const int64_t* __restrict__ offset_ptr,
                                SingleForwardArgs a) {
-    // [0] the mean's sum, [1] the variance's: one float per wave of the row
-    // (direct), or one per vector of the block's rows (exchange, at most four
-    // waves).
-    constexpr int kShared = Path == SumPath::kExchange ? V * 4 * kWaveSize : kSingleMaxParts;
-    __shared__ float shared[2][kShared];
+    // [0] the mean's sum, [1] the variance's.
+    __shared__ float shared[2][single_shared_size(Path, V)];
     // Keep bits of the reference's stream, 64 columns each (at most 1024
     // columns, so at most 16 per row, and at most four rows per block).
     __shared__ uint64_t keep[4][16];
@@ -496,7 +512,7 @@ void rln_single_forward_kernel(const float* x_rows, const B* branch_rows, int ro
     const int64_t row = valid ? team_row : 0;
     const int64_t count = valid ? hidden : 0;
     const int64_t base = row * hidden;
-    const int row_shared = Path == SumPath::kExchange ? group * V * parts * kWaveSize : 0;
+    const int row_shared = single_shared_first(Path, V, parts, group);
 
     // The Philox key and position first: the draws hang on them, and under
     // graph capture they come from memory.
@@ -796,10 +812,7 @@ void rln_single_backward_kernel(const float* updated, const GY* grad_normalized,
                                  static_cast<int>(end - begin));
         return;
     }
-    // Direct: the wave totals of both sums; exchange: both of every vector of
-    // the block's rows (at most four waves).
-    constexpr int kShared = Path == SumPath::kExchange ? 4 * kWaveSize : kSingleMaxWaves;
-    __shared__ float2 shared[kShared];
+    __shared__ float2 shared[single_shared_size(Path, V)];  // both sums
     const int lane = threadIdx.x & (kWaveSize - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int parts = split.parts();
@@ -852,8 +865,8 @@ void rln_single_backward_kernel(const float* updated, const GY* grad_normalized,
             (q.x * xhat[v].x + q.y * xhat[v].y) + (q.z * xhat[v].z + q.w * xhat[v].w);
     }
     const float2 totals = single_pair_sum<V, Path>(
-        q_slots, qx_slots, shared + group * parts * (Path == SumPath::kExchange ? kWaveSize : 1),
-        parts, part, split.order());
+        q_slots, qx_slots, shared + single_shared_first(Path, V, parts, group), parts, part,
+        split.order());
     const float mean_q = totals.x * a.inv_hidden;
     const float mean_qx = totals.y * a.inv_hidden;
     const rsrc_t grad_x_out = output_range(a.grad_x, base, count);

@@ -1,0 +1,47 @@
+"""The host rules of the single-step kernels (csrc/rln_single.h), on the CPU.
+
+tests/sanitize/rln_rules.hip compiles the rules with the host sanitizers and
+answers queries about them; nothing reaches a device.
+"""
+
+import os
+import subprocess
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent / "sanitize"
+HIDDEN = range(128, 8193, 64)
+
+
+@pytest.fixture(scope="module")
+def ask():
+    """ask(queries): one list of integers per query line."""
+    if not Path("/opt/rocm/bin/hipcc").exists():
+        pytest.skip("no hipcc")
+    build = subprocess.run(["make", "-s", "-C", str(HERE), "rln_rules"], capture_output=True,
+                           text=True, timeout=600)
+    assert build.returncode == 0, build.stdout + build.stderr
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=1",
+               UBSAN_OPTIONS="halt_on_error=1:print_stacktrace=1")
+
+    def run(queries):
+        lines = [" ".join(str(int(v)) if not isinstance(v, str) else v for v in query)
+                 for query in queries]
+        result = subprocess.run([str(HERE / "rln_rules")], input="\n".join(lines) + "\n",
+                                capture_output=True, text=True, timeout=300, env=env)
+        assert result.returncode == 0, result.stderr
+        answers = [[int(v) for v in line.split()] for line in result.stdout.splitlines()]
+        assert len(answers) == len(lines)
+        return answers
+
+    return run
+
+
+def test_row_sums_stay_inside_their_lds_array(ask):
+    """Every row of every split reads its sums from inside the block's array
+    (rows of 1025-1216 columns share a block of four waves, two rows of two)."""
+    queries = [("lds", pass_, rows, hidden) for pass_ in (0, 1) for hidden in HIDDEN
+               for rows in (1, 5, 2048, 8192, 8193, 12291, 65536)]
+    for query, (size, end) in zip(queries, ask(queries)):
+        assert end <= size, query
