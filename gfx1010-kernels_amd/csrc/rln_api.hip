@@ -130,14 +130,6 @@ bool aligned_to(const void* pointer, uintptr_t alignment) {
     return pointer == nullptr || (reinterpret_cast<uintptr_t>(pointer) & (alignment - 1)) == 0;
 }
 
-// Whether two device ranges share a byte (null: no range).
-bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
-    const uintptr_t first = reinterpret_cast<uintptr_t>(a);
-    const uintptr_t second = reinterpret_cast<uintptr_t>(b);
-    return a != nullptr && b != nullptr && first < second + static_cast<uintptr_t>(b_bytes)
-        && second < first + static_cast<uintptr_t>(a_bytes);
-}
-
 // Mirrors the reference's conversion of the double probability
 // (csrc/residual_layer_norm_kernel.hip:893-899, :1883-1886).
 struct DropoutConstants {
@@ -482,23 +474,7 @@ int backward_launches(
         && aligned_to(grad_normalized, vector_alignment(grad_normalized_dtype))
         && aligned_to(updated, 16) && aligned_to(weight, 16) && aligned_to(grad_x, 16)
         && aligned_to(grad_branch, vector_alignment(branch_dtype));
-    // The single-step backward's slab blocks read `updated` and
-    // grad_normalized beside the row blocks' stores: gradients written over
-    // them take the walking kernels, which read each row once, before its
-    // stores.
-    const int64_t bytes = rows * hidden * 4;
-    const auto written = [&](const void* input, int64_t input_bytes) {
-        return overlap(input, input_bytes, grad_x, bytes)
-            || overlap(input, input_bytes, grad_branch,
-                       branch_dtype == RLN_DTYPE_F32 ? bytes : bytes / 2);
-    };
-    const bool single = single_backward(rows, hidden, grad_normalized_dtype)
-        && !(partials && !single_partials(rows, hidden))
-        && !(parameters
-             && (written(updated, bytes)
-                 || written(grad_normalized,
-                            grad_normalized_dtype == RLN_DTYPE_F32 ? bytes : bytes / 2)
-                 || written(mean, rows * 4) || written(rstd, rows * 4)));
+    const bool single = takes_single_backward(a, hidden, branch_dtype, grad_normalized_dtype);
     if (single) {
         status = launch_single_backward(a, hidden, branch_dtype, grad_normalized_dtype, aligned);
     } else {

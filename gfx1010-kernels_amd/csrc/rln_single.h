@@ -213,6 +213,41 @@ inline bool single_partials(int64_t rows, int64_t hidden) {
     return rows <= (hidden == 128 ? 4096 : 64 * kBackwardMaxBlocks);
 }
 
+// Whether two device ranges share a byte (null: no range).
+inline bool ranges_overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+    const uintptr_t first = reinterpret_cast<uintptr_t>(a);
+    const uintptr_t second = reinterpret_cast<uintptr_t>(b);
+    return a != nullptr && b != nullptr && first < second + static_cast<uintptr_t>(b_bytes)
+        && second < first + static_cast<uintptr_t>(a_bytes);
+}
+
+// Whether a backward writes grad_x or grad_branch over `updated`,
+// grad_normalized, mean or rstd.
+inline bool gradients_over_inputs(const BackwardArgs& a, int64_t hidden, int branch_dtype,
+                                  int grad_normalized_dtype) {
+    const int64_t bytes = a.rows * hidden * 4;
+    const auto sized = [&](int dtype) { return dtype == RLN_DTYPE_F32 ? bytes : bytes / 2; };
+    const auto written = [&](const void* input, int64_t input_bytes) {
+        return ranges_overlap(input, input_bytes, a.grad_x, bytes)
+            || ranges_overlap(input, input_bytes, a.grad_branch, sized(branch_dtype));
+    };
+    return written(a.updated, bytes) || written(a.grad_normalized, sized(grad_normalized_dtype))
+        || written(a.mean, a.rows * 4) || written(a.rstd, a.rows * 4);
+}
+
+// Whether a backward launch runs single-step. Its slab blocks read `updated`
+// and grad_normalized beside the row blocks' stores, so gradients written over
+// what they read take the walking kernels, which read each row once, before
+// its stores. (The size rules come first: sizes in bytes are then small, while
+// the C ABI accepts row counts whose bytes overflow int64.)
+inline bool takes_single_backward(const BackwardArgs& a, int64_t hidden, int branch_dtype,
+                                  int grad_normalized_dtype) {
+    return single_backward(a.rows, hidden, grad_normalized_dtype)
+        && !((a.flags & kPartials) && !single_partials(a.rows, hidden))
+        && !((a.flags & kParameters)
+             && gradients_over_inputs(a, hidden, branch_dtype, grad_normalized_dtype));
+}
+
 // A block's LDS array of row sums: its length, where the sums of the block's
 // row `group` begin, and how many elements from there its lanes read. Direct:
 // one per wave; the lanes read kSingleMaxParts of them in a fixed loop and drop

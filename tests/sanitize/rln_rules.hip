@@ -7,6 +7,12 @@
 //   lds PASS ROWS HIDDEN    length of the block's array of row sums, and one
 //                           past the last element its rows read (PASS 0:
 //                           forward, 1: backward)
+//   backward ROWS HIDDEN BRANCH GRAD_NORMALIZED FLAGS OVER
+//                           1 if a backward with these dtypes and flags
+//                           (kHasGradUpdated, ... of rln_device.h) runs
+//                           single-step; OVER: what shares its memory, 0 nothing,
+//                           1 grad_x and updated, 2 grad_x and grad_normalized,
+//                           3 grad_branch and updated, 4 grad_branch and mean
 #include <cstdio>
 #include <iostream>
 #include <sstream>
@@ -24,6 +30,25 @@ void lds(int64_t rows, int64_t hidden) {
     std::printf("%d %d\n", rln::single_shared_size(s.path, s.vectors), end);
 }
 
+void* at(int64_t tebibytes) {
+    return reinterpret_cast<void*>(static_cast<uintptr_t>(tebibytes) << 40);
+}
+
+bool backward(int64_t rows, int64_t hidden, int branch, int grad_normalized, int flags, int over) {
+    rln::BackwardArgs a{};
+    a.rows = rows;
+    a.flags = flags;
+    a.grad_updated = static_cast<const float*>((flags & rln::kHasGradUpdated) ? at(1) : nullptr);
+    a.grad_normalized = (flags & rln::kHasGradNormalized) ? at(2) : nullptr;
+    a.updated = static_cast<const float*>(at(3));
+    a.weight = static_cast<const float*>(at(4));
+    a.mean = static_cast<const float*>(at(5));
+    a.rstd = static_cast<const float*>(at(6));
+    a.grad_x = static_cast<float*>(at(over == 1 ? 3 : over == 2 ? 2 : 7));
+    a.grad_branch = at(over == 3 ? 3 : over == 4 ? 5 : 8);
+    return rln::takes_single_backward(a, hidden, branch, grad_normalized);
+}
+
 }  // namespace
 
 int main() {
@@ -37,6 +62,13 @@ int main() {
             in >> pass >> rows >> hidden;
             pass == 0 ? lds<rln::Pass::kForward>(rows, hidden)
                       : lds<rln::Pass::kBackward>(rows, hidden);
+        } else if (query == "backward") {
+            int64_t rows = 0, hidden = 0;
+            int branch = 0, grad_normalized = 0, flags = 0, over = 0;
+            in >> rows >> hidden >> branch >> grad_normalized >> flags >> over;
+            std::printf("%d\n", backward(rows, hidden, branch, grad_normalized, flags, over));
+        } else {
+            query.clear();
         }
         if (in.fail() || query.empty()) {
             std::fprintf(stderr, "bad query: %s\n", line.c_str());

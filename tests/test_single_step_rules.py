@@ -45,3 +45,27 @@ def test_row_sums_stay_inside_their_lds_array(ask):
                for rows in (1, 5, 2048, 8192, 8193, 12291, 65536)]
     for query, (size, end) in zip(queries, ask(queries)):
         assert end <= size, query
+
+
+F32, F16, BF16 = 0, 1, 2
+GRAD_UPDATED, GRAD_NORMALIZED, DROPOUT, PARAMETERS, PARTIALS = 1, 2, 4, 8, 16
+EVERYTHING = GRAD_UPDATED | GRAD_NORMALIZED | DROPOUT | PARAMETERS
+
+
+def test_row_counts_whose_bytes_overflow(ask):
+    """The C ABI accepts every rows * hidden that fits int64; the choice of the
+    backward's kernel must not overflow on the bytes of such tensors."""
+    queries = [("backward", (2**63 - 1) // hidden, hidden, F32, F32, flags, over)
+               for hidden in (128, 768, 8192) for over in range(5)
+               for flags in (EVERYTHING, EVERYTHING | PARTIALS)]
+    assert ask(queries) == [[0]] * len(queries)
+
+
+@pytest.mark.parametrize("hidden", [128, 768, 2880])
+def test_gradients_over_inputs_walk(ask, hidden):
+    """Gradients in the memory of what the slab blocks read take the walking
+    kernels; without weight/bias sums there are no slab blocks."""
+    for over in range(5):
+        answers = ask([("backward", 100, hidden, F16, F32, EVERYTHING, over),
+                       ("backward", 100, hidden, F16, F32, EVERYTHING & ~PARAMETERS, over)])
+        assert answers == [[int(over == 0)], [1]]
