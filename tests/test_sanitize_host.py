@@ -32,3 +32,14 @@ def test_validation_paths_run_clean_under_host_sanitizers():
                          timeout=300, env=env)
     assert run.returncode == 0, run.stdout + run.stderr
     assert run.stdout.strip().splitlines()[-1] == "ok", run.stdout + run.stderr
+
+
+@pytest.mark.parametrize("target", ["rln_api_sanitized.o", "rln_rules"])
+@pytest.mark.parametrize("header", ["gfx1010-kernels_amd/csrc/rln_single.h",
+                                    "gfx1010-kernels_amd/csrc/rln_device.h", "include/rln.h"])
+def test_sanitized_builds_depend_on_their_headers(target, header):
+    """A change to a header that a target includes rebuilds it: a stale object
+    would let the sanitizer tests pass on code that is gone."""
+    dry = subprocess.run(["make", "-n", "-W", str(HERE.parents[1] / header), "-C", str(HERE),
+                          target], capture_output=True, text=True, timeout=60)
+    assert dry.returncode == 0 and f"-o {target}" in dry.stdout, dry.stdout + dry.stderr
