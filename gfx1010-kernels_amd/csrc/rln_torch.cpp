@@ -214,29 +214,44 @@ int dtype_of(at::ScalarType type) {
     return RLN_DTYPE_F32;
 }
 
-// Outputs and scratch, straight from the caching allocator. at::empty would go
+// Whether something on this thread looks on at, or takes over, every operator:
+// a TorchDispatchMode (FakeTensorMode among them), a functorch transform, a
+// trace. Its dispatch key is then in the thread's included set.
+bool dispatch_watched() {
+    return !(c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty();
+}
+
+// Outputs and scratch, straight from the caching allocator. at::empty goes
 // through the dispatcher and, under torch.use_deterministic_algorithms(True),
-// fill every new tensor with NaN (torch.utils.deterministic.
+// fills every new tensor with NaN (torch.utils.deterministic.
 // fill_uninitialized_memory): seven extra passes per training step over
 // memory that the kernels overwrite whole. Measured on MI355X: eager forward +
 // backward of [65536, 1024], fp16 branch, in deterministic mode 499.5 -> 349.9
-// us; a no_grad call of [8, 768] (bound by the host) 8.40 -> 7.83 us.
+// us; a no_grad call of [8, 768] (bound by the host) 8.40 -> 7.83 us. A watched
+// thread keeps at::empty: a memory-counting mode sees the allocations, and a
+// FakeTensorMode or functorch transform around tensors of real memory is
+// refused as by any operator that asks for their addresses.
 at::Tensor empty_device(at::IntArrayRef sizes, at::ScalarType type, const at::Device& device) {
+    if (dispatch_watched()) {
+        return at::empty(sizes, at::TensorOptions(device).dtype(type));
+    }
     return at::Tensor(at::detail::empty_cuda(sizes, type, device, std::nullopt));
 }
 
-// at::empty_like of a contiguous tensor. Contiguity says nothing about the
-// strides of dimensions of size 1, which at::empty_like keeps: those that are
-// not the plain row-major ones still go through it.
+// at::empty_like of a contiguous tensor. What it takes over from `like` goes
+// through it: dimension names, a __torch_dispatch__ subclass, and the strides of
+// dimensions of size 1, of which contiguity says nothing, where they are not
+// the plain row-major ones.
 at::Tensor empty_device_like(const at::Tensor& like, at::ScalarType type) {
+    bool plain = !dispatch_watched() && !like.has_names()
+        && !like.key_set().has(c10::DispatchKey::Python);
     int64_t stride = 1;
-    for (int64_t i = like.dim() - 1; i >= 0; --i) {
-        if (like.stride(i) != stride) {
-            return at::empty_like(like, like.options().dtype(type));
-        }
+    for (int64_t i = like.dim() - 1; plain && i >= 0; --i) {
+        plain = like.stride(i) == stride;
         stride *= like.size(i);
     }
-    return empty_device(like.sizes(), type, like.device());
+    return plain ? empty_device(like.sizes(), type, like.device())
+                 : at::empty_like(like, like.options().dtype(type));
 }
 
 // Row statistics and dropout mask of one forward call kept in a single

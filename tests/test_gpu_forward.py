@@ -6,6 +6,8 @@ train with dropout, the reference's row-count boundaries
 element-access path (tests/test_residual_layer_norm_vectorized.py:96-164).
 """
 
+import warnings
+
 import pytest
 import torch
 
@@ -246,3 +248,70 @@ def test_outputs_follow_empty_like_and_are_written_whole(strides, deterministic)
         results.append([*outputs, *gradients])
     for first, second in zip(*results):
         assert torch.isfinite(first).all() and torch.equal(first, second)
+
+
+def _plain_call(grad):
+    generator = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(2, 5, 128, device="cuda", generator=generator)
+    branch = torch.randn(2, 5, 128, device="cuda", generator=generator)
+    weight, bias = torch.rand(2, 128, device="cuda", generator=generator)
+    return x.requires_grad_(grad), branch, weight, bias
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_outputs_keep_dimension_names(grad):
+    """Outputs take x's dimension names, as torch.empty_like does."""
+    x, branch, weight, bias = _plain_call(False)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        named = x.refine_names("N", "T", "C").requires_grad_(grad)
+    for outputs in (residual_layer_norm(named, branch, weight, bias, 0.0, 1e-5, True,
+                                        implementation=implementation)
+                    for implementation in ("gfx950", "auto")):
+        assert [t.names for t in outputs] == [("N", "T", "C")] * 2
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_dispatch_modes_see_the_allocations(grad):
+    """A TorchDispatchMode that counts memory sees every tensor a call and its
+    backward allocate."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Allocations(TorchDispatchMode):
+        elements = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            if func.overloadpacket in (torch.ops.aten.empty, torch.ops.aten.empty_like):
+                self.elements += out.numel()
+            return out
+
+    x, branch, weight, bias = _plain_call(grad)
+    ones = torch.ones_like(x)
+    with Allocations() as mode:
+        outputs = residual_layer_norm(x, branch, weight, bias, 0.1, 1e-5, True,
+                                      implementation="gfx950")
+        forward = mode.elements
+        if grad:
+            torch.autograd.grad(outputs, [x], [ones, ones])
+    # Both outputs, and mean, rstd (64-element rows) and the mask in one tensor.
+    assert forward == 2 * x.numel() + 64 + 64 + x.numel() // 32
+    assert mode.elements - forward == (2 * x.numel() if grad else 0)
+
+
+def test_transforms_around_real_tensors_are_refused():
+    """A functorch transform or FakeTensorMode around a call on closed-over real
+    tensors is refused, not run beside it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    x, branch, weight, bias = _plain_call(False)
+
+    def call():
+        return residual_layer_norm(x, branch, weight, bias, 0.0, 1e-5, False,
+                                   implementation="gfx950")[1]
+
+    with pytest.raises(RuntimeError, match="data pointer|not allocated"):
+        torch.func.grad(lambda scale: (call() * scale).sum())(torch.ones((), device="cuda"))
+    with pytest.raises(RuntimeError, match="not allocated"):
+        with FakeTensorMode(allow_non_fake_inputs=True):
+            call()
