@@ -335,7 +335,7 @@ int rln_forward(
         && aligned_to(updated, 16)
         && aligned_to(normalized, vector_alignment(normalized_dtype))
         && aligned_to(branch, vector_alignment(branch_dtype));
-    if (single_forward(rows, hidden, drop.active)) {
+    if (single_forward(rows, hidden, drop.active, aligned)) {
         return launch_single_forward(a, hidden, branch_dtype, normalized_dtype, aligned);
     }
     return with_shape<Pass::kForward>(hidden, rows, [&](auto shape) {
@@ -474,7 +474,8 @@ int backward_launches(
         && aligned_to(grad_normalized, vector_alignment(grad_normalized_dtype))
         && aligned_to(updated, 16) && aligned_to(weight, 16) && aligned_to(grad_x, 16)
         && aligned_to(grad_branch, vector_alignment(branch_dtype));
-    const bool single = takes_single_backward(a, hidden, branch_dtype, grad_normalized_dtype);
+    const bool single =
+        takes_single_backward(a, hidden, branch_dtype, grad_normalized_dtype, aligned);
     if (single) {
         status = launch_single_backward(a, hidden, branch_dtype, grad_normalized_dtype, aligned);
     } else {

@@ -124,8 +124,20 @@ SingleSplit single_split(int64_t hidden, int64_t rows) {
 // [8192, 128] 7.0 -> 7.8; [655, 1600] 5.6 -> 5.1, [993, 1600] 6.2 -> 6.4).
 // Without dropout, rows above 4096 columns only for a few rows ([1, 8192]
 // 5.0 -> 4.7 us, [32, 8192] 5.3 -> 5.6; with dropout [128, 8192] 7.2 -> 6.7).
-inline bool single_forward(int64_t rows, int64_t hidden, bool dropout) {
+//
+// Misaligned tensors (element accesses) up to 384 K elements (512 K for 512-1024
+// columns) of rows of at most 4096 columns: from there four times the access
+// instructions per lane cost more than the walk (us, walking -> single-step: [341,
+// 768] with dropout 8.3 -> 5.1, [512, 1024] 10.9 -> 7.0, [64, 4096] 7.7 -> 6.4; past
+// the lines [257, 2880] fp16 8.7 -> 10.1, [1927, 1088] 18.5 -> 21.9), and above 4096
+// columns it gains nothing at any size ([12, 5120] without dropout 5.7 -> 6.2, [64,
+// 8192] with it 9.4 -> 10.3).
+inline bool single_forward(int64_t rows, int64_t hidden, bool dropout, bool aligned) {
     const int64_t elements = rows * hidden;
+    if (!aligned) {
+        return hidden <= 4096
+            && elements <= (hidden >= 512 && hidden <= 1024 ? 512 << 10 : 384 << 10);
+    }
     if (hidden > 4096 && !dropout) {
         return elements <= (1 << 17);
     }
@@ -167,19 +179,60 @@ __device__ __forceinline__ void row_handoff(int parts) {
 // that alternate fit the 256 MB Infinity Cache by half (forward + backward
 // over three batches 39.9 against 41.6 us, over eight 41.9 against 40.1; with
 // 16-bit gradients 39.2 -> 37.0 over three).
-inline bool single_backward(int64_t rows, int64_t hidden, int grad_normalized_dtype) {
-    const int64_t elements = rows * hidden;
-    if (grad_normalized_dtype == RLN_DTYPE_F32 && rows >= 7168
-        && backward_twelve_waves(hidden, rows)) {
+//
+// Misaligned tensors (element accesses) have lines of their own. At 320-768
+// columns, whose rows hold one slot per lane, they are the same ([5461, 768] 33.7
+// -> 21.8, [6553, 640] 36.5 -> 22.1); elsewhere the slab blocks' second read costs
+// four times the instructions. With weight/bias sums: [5792, 128] 11.1 -> 8.8, [772,
+// 960] 14.0 -> 8.7, [926, 1600] 17.5 -> 15.5, [252, 4160] 20.8 -> 10.8, [337, 6208] 34.6
+// -> 20.9; past the lines [11585, 128] fp32 17.4 -> 19.1, [4369, 960] fp32 40.6 ->
+// 49.7, [712, 4160] 29.6 -> 33.4, [675, 6208] fp32 51.1 -> 60.2, [682, 6144] fp32 42.5 ->
+// 63.1. Without sums, where only the row chains can gain: [204, 1280] 5.8 -> 4.7,
+// [579, 1280] 8.3 -> 9.6, and rows of 2433-6144 columns lose at every size ([21,
+// 3072] 4.4 -> 4.6, [482, 3072] 12.2 -> 14.8). Deterministic sums are the same bits
+// for tensors of any alignment, so their line does not ask for it.
+struct SingleBackwardCall {
+    int64_t rows;
+    int64_t hidden;
+    int grad_normalized_dtype;
+    bool sums;      // weight and bias sums, by atomics or ...
+    bool partials;  // ... through partials in the workspace
+    bool aligned;   // vector accesses
+};
+
+inline int64_t single_backward_most(const SingleBackwardCall& c) {
+    constexpr int64_t K = 1 << 10;
+    constexpr int64_t M = 1 << 20;
+    struct Misaligned {
+        int64_t hidden;  // rows of up to so many columns
+        int64_t sums;    // elements
+        int64_t none;
+    };
+    constexpr Misaligned kMisaligned[] = {
+        {256, M, 256 * K},  {768, 12 * M, 12 * M}, {1024, M, 384 * K},           {2432, M, 512 * K},
+        {4096, M, 0},       {6144, 1536 * K, 0},   {kMaxHidden, 3 * M, 2 * M},
+    };
+    if (!c.aligned && !c.partials) {
+        for (const Misaligned& line : kMisaligned) {
+            if (c.hidden <= line.hidden) {
+                return c.sums ? line.sums : line.none;
+            }
+        }
+    }
+    return c.hidden == 128   ? 4 * M
+        : c.hidden == 256    ? 8 * M
+        : c.hidden <= 1024   ? 12 * M
+        : c.hidden < 4096    ? 6 * M
+        : c.hidden <= 6144   ? 8 * M
+                             : 16 * M;
+}
+
+inline bool single_backward(const SingleBackwardCall& c) {
+    if (c.grad_normalized_dtype == RLN_DTYPE_F32 && c.rows >= 7168
+        && backward_twelve_waves(c.hidden, c.rows)) {
         return false;
     }
-    const int64_t most = hidden == 128 ? 1 << 22
-        : hidden == 256               ? 1 << 23
-        : hidden <= 1024              ? 12 << 20
-        : hidden < 4096               ? 6 << 20
-        : hidden <= 6144              ? 1 << 23
-                                      : 1 << 24;
-    return elements <= most;
+    return c.rows * c.hidden <= single_backward_most(c);
 }
 
 // Rows of one chunk: its blocks run on one XCD, and its slab blocks read again
@@ -241,11 +294,12 @@ inline bool gradients_over_inputs(const BackwardArgs& a, int64_t hidden, int bra
 // its stores. (The size rules come first: sizes in bytes are then small, while
 // the C ABI accepts row counts whose bytes overflow int64.)
 inline bool takes_single_backward(const BackwardArgs& a, int64_t hidden, int branch_dtype,
-                                  int grad_normalized_dtype) {
-    return single_backward(a.rows, hidden, grad_normalized_dtype)
-        && !((a.flags & kPartials) && !single_partials(a.rows, hidden))
-        && !((a.flags & kParameters)
-             && gradients_over_inputs(a, hidden, branch_dtype, grad_normalized_dtype));
+                                  int grad_normalized_dtype, bool aligned) {
+    const bool sums = (a.flags & kParameters) != 0;
+    const bool partials = (a.flags & kPartials) != 0;
+    return single_backward({a.rows, hidden, grad_normalized_dtype, sums, partials, aligned})
+        && !(partials && !single_partials(a.rows, hidden))
+        && !(sums && gradients_over_inputs(a, hidden, branch_dtype, grad_normalized_dtype));
 }
 
 // A block's LDS array of row sums: its length, where the sums of the block's

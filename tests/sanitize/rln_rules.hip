@@ -7,7 +7,10 @@
 //   lds PASS ROWS HIDDEN    length of the block's array of row sums, and one
 //                           past the last element its rows read (PASS 0:
 //                           forward, 1: backward)
-//   backward ROWS HIDDEN BRANCH GRAD_NORMALIZED FLAGS OVER
+//   forward ROWS HIDDEN DROPOUT ALIGNED
+//                           1 if a forward runs single-step, and 1 if it writes
+//                           through
+//   backward ROWS HIDDEN BRANCH GRAD_NORMALIZED FLAGS OVER ALIGNED
 //                           1 if a backward with these dtypes and flags
 //                           (kHasGradUpdated, ... of rln_device.h) runs
 //                           single-step; OVER: what shares its memory, 0 nothing,
@@ -34,7 +37,8 @@ void* at(int64_t tebibytes) {
     return reinterpret_cast<void*>(static_cast<uintptr_t>(tebibytes) << 40);
 }
 
-bool backward(int64_t rows, int64_t hidden, int branch, int grad_normalized, int flags, int over) {
+bool backward(int64_t rows, int64_t hidden, int branch, int grad_normalized, int flags, int over,
+              bool aligned) {
     rln::BackwardArgs a{};
     a.rows = rows;
     a.flags = flags;
@@ -46,7 +50,7 @@ bool backward(int64_t rows, int64_t hidden, int branch, int grad_normalized, int
     a.rstd = static_cast<const float*>(at(6));
     a.grad_x = static_cast<float*>(at(over == 1 ? 3 : over == 2 ? 2 : 7));
     a.grad_branch = at(over == 3 ? 3 : over == 4 ? 5 : 8);
-    return rln::takes_single_backward(a, hidden, branch, grad_normalized);
+    return rln::takes_single_backward(a, hidden, branch, grad_normalized, aligned);
 }
 
 }  // namespace
@@ -65,8 +69,16 @@ int main() {
         } else if (query == "backward") {
             int64_t rows = 0, hidden = 0;
             int branch = 0, grad_normalized = 0, flags = 0, over = 0;
-            in >> rows >> hidden >> branch >> grad_normalized >> flags >> over;
-            std::printf("%d\n", backward(rows, hidden, branch, grad_normalized, flags, over));
+            bool aligned = true;
+            in >> rows >> hidden >> branch >> grad_normalized >> flags >> over >> aligned;
+            std::printf("%d\n",
+                        backward(rows, hidden, branch, grad_normalized, flags, over, aligned));
+        } else if (query == "forward") {
+            int64_t rows = 0, hidden = 0;
+            bool dropout = false, aligned = true;
+            in >> rows >> hidden >> dropout >> aligned;
+            std::printf("%d %d\n", rln::single_forward(rows, hidden, dropout, aligned),
+                        rln::forward_write_through(rows, hidden, aligned));
         } else {
             query.clear();
         }

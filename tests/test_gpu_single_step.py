@@ -146,3 +146,22 @@ def test_gradients_written_over_their_inputs(rows, hidden, over):
     assert torch.equal(results[0][1], results[1][1])
     # Two fp32 orders of sums over at most 100 values of order one.
     assert torch.allclose(results[0][2], results[1][2], rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("rows,hidden", [(341, 768), (512, 1024), (64, 4096), (257, 2880), (5792, 128),
+                                         (11585, 128), (772, 960), (4369, 960), (252, 4160),
+                                         (712, 4160), (337, 6208), (675, 6208)])
+def test_misaligned_launches_match_aligned_ones(rows, hidden):
+    """Both sides of the lines from which element accesses walk: row outputs are
+    the aligned launch's bits, weight/bias sums at the parity bar."""
+    from test_gpu_schedules import ROW_OUTPUTS, assert_same_bits, check_parameter_sums, empty, run
+
+    print(f"[single step] misaligned rows={rows} H={hidden}", flush=True)
+    inputs, grads = device_inputs(rows, hidden, torch.bfloat16, seed=rows + hidden)
+    aligned_case = (*inputs, *grads)
+    shifted_case = tuple(empty(t.shape, t.dtype, shift=1).copy_(t) for t in aligned_case)
+    aligned = run(aligned_case, rows, torch.float32, 0.1, False)
+    shifted = run(shifted_case, rows, torch.float32, 0.1, False, shift=1)
+    for name in (*ROW_OUTPUTS, "mask"):
+        assert_same_bits(shifted[name], aligned[name], name)
+    check_parameter_sums(shifted, grads[1], rows)

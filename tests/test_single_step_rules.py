@@ -55,7 +55,7 @@ EVERYTHING = GRAD_UPDATED | GRAD_NORMALIZED | DROPOUT | PARAMETERS
 def test_row_counts_whose_bytes_overflow(ask):
     """The C ABI accepts every rows * hidden that fits int64; the choice of the
     backward's kernel must not overflow on the bytes of such tensors."""
-    queries = [("backward", (2**63 - 1) // hidden, hidden, F32, F32, flags, over)
+    queries = [("backward", (2**63 - 1) // hidden, hidden, F32, F32, flags, over, 1)
                for hidden in (128, 768, 8192) for over in range(5)
                for flags in (EVERYTHING, EVERYTHING | PARTIALS)]
     assert ask(queries) == [[0]] * len(queries)
@@ -66,6 +66,45 @@ def test_gradients_over_inputs_walk(ask, hidden):
     """Gradients in the memory of what the slab blocks read take the walking
     kernels; without weight/bias sums there are no slab blocks."""
     for over in range(5):
-        answers = ask([("backward", 100, hidden, F16, F32, EVERYTHING, over),
-                       ("backward", 100, hidden, F16, F32, EVERYTHING & ~PARAMETERS, over)])
+        answers = ask([("backward", 100, hidden, F16, F32, EVERYTHING, over, 1),
+                       ("backward", 100, hidden, F16, F32, EVERYTHING & ~PARAMETERS, over, 1)])
         assert answers == [[int(over == 0)], [1]]
+
+
+# (rows, hidden, branch, grad_normalized, flags, single-step?) on both sides of
+# lines beside which rln_single.h gives both sides' times.
+NONE = EVERYTHING & ~PARAMETERS
+MISALIGNED = [
+    (5792, 128, F16, F32, EVERYTHING, 1), (11585, 128, F32, F32, EVERYTHING, 0),
+    (5461, 768, F32, F32, EVERYTHING, 1), (6553, 640, BF16, BF16, EVERYTHING, 1),
+    (772, 960, F16, F32, EVERYTHING, 1), (4369, 960, F32, F32, EVERYTHING, 0),
+    (252, 4160, F16, F32, EVERYTHING, 1), (712, 4160, F16, F32, EVERYTHING, 0),
+    (682, 6144, F32, F32, EVERYTHING, 0), (337, 6208, F32, F32, EVERYTHING, 1),
+    (675, 6208, F32, F32, EVERYTHING, 0),
+    (204, 1280, F16, F32, NONE, 1), (579, 1280, F16, F32, NONE, 0),
+    (21, 3072, F16, F32, NONE, 0), (482, 3072, F16, F32, NONE, 0),
+]
+
+
+def test_misaligned_backward_lines(ask):
+    """Element accesses take the walking backward where it is the faster one."""
+    assert ask([("backward", *case[:5], 0, 0) for case in MISALIGNED]) \
+        == [[case[5]] for case in MISALIGNED]
+
+
+def test_misaligned_forward_lines(ask):
+    """Element accesses: single-step for small launches of up to 4096 columns,
+    write-through below 2^23 elements at every row length."""
+    cases = [(341, 768, 1, 1, 1), (1365, 768, 1, 0, 1), (512, 1024, 1, 1, 1), (64, 4096, 1, 1, 1),
+             (257, 2880, 1, 0, 1), (1927, 1088, 1, 0, 1),
+             (12, 5120, 0, 0, 1), (64, 8192, 1, 0, 1), (7414, 1600, 1, 0, 0),
+             (10485, 1600, 1, 0, 0), (65536, 256, 1, 0, 0), (5242, 1600, 1, 0, 1)]
+    assert ask([("forward", *case[:3], 0) for case in cases]) == [list(case[3:]) for case in cases]
+
+
+def test_deterministic_route_ignores_alignment(ask):
+    """Deterministic weight/bias sums are the same bits for tensors of any
+    alignment: the kernel that groups them is chosen without it."""
+    queries = [("backward", rows, hidden, F16, F32, EVERYTHING | PARTIALS, 0)
+               for hidden in HIDDEN for rows in (1, 60, 300, 1000, 3000, 9000, 20000)]
+    assert ask([(*q, 0) for q in queries]) == ask([(*q, 1) for q in queries])
