@@ -195,6 +195,7 @@ struct SingleBackwardCall {
     int64_t rows;
     int64_t hidden;
     int grad_normalized_dtype;
+    bool has_grad_normalized;
     bool sums;      // weight and bias sums, by atomics or ...
     bool partials;  // ... through partials in the workspace
     bool aligned;   // vector accesses
@@ -224,7 +225,49 @@ inline int64_t single_backward_most(const SingleBackwardCall& c) {
         : c.hidden <= 1024   ? 12 * M
         : c.hidden < 4096    ? 6 * M
         : c.hidden <= 6144   ? 8 * M
-                             : 16 * M;
+        : c.hidden <= 7936 || c.sums ? 16 * M
+                                     : 3 * M;
+}
+
+// A backward without weight/bias sums (frozen parameters, or no grad_normalized)
+// has no atomics to save, and the walk of few rows is short: where its whole
+// grid of one block per CU is (nearly) full in its first or second row step,
+// single-step blocks lose up to a quarter. Measured (us, walking ->
+// single-step), frozen parameters unless said otherwise:
+//  * eight-wave rows of 2433-6144 columns (one row per block and step): up to
+//    256 rows [241, 3072] 5.1 -> 4.5, above [482, 3072] 7.1 -> 7.7, [512, 4096] 8.1 ->
+//    9.1, [682, 6144] fp32 17.2 -> 21.0 (forward and backward [682, 3072] 18.2 ->
+//    20.3); without grad_normalized, whose walk is shorter, up to 2^19 elements
+//    of 2433-5120 columns too ([42, 3072] 3.1 -> 3.4, [148, 2496] 3.6 -> 3.9; [241,
+//    3072] 4.8 -> 4.3, [85, 6144] 5.3 -> 4.7);
+//  * four-wave rows of 1217-2048 columns, 768 to a step: [579, 1280] 5.1 -> 5.4,
+//    [655, 1600] 5.8 -> 6.3, [724, 2048] 6.8 -> 7.9, [1170, 1792] 9.1 -> 9.7;
+//    and beside them [512, 2048] 5.8 -> 5.7, [926, 1600] 8.3 -> 7.3; of 2049-2432
+//    columns, 512 to a step, its second: [862, 2432] 9.1 -> 9.4 (forward and
+//    backward [609, 2432] 16.3 -> 17.4);
+//  * rows of 128-256 columns without grad_normalized in the first step: [4096, 128]
+//    3.7 -> 4.0, [5792, 128] 5.3 -> 4.5;
+//  * rows of 8000-8192 columns lose from 3 M elements ([362, 8192] 18.1 -> 13.7, [512,
+//    8192] fp32 22.1 -> 25.0, [1448, 8192] 45.5 -> 50.8), shorter ones up to 7936 do not
+//    ([1170, 7168] 33.5 -> 34.3).
+inline bool walk_without_sums(const SingleBackwardCall& c) {
+    const ShapeInfo info = shape_info(c.hidden, Pass::kBackward, c.rows);
+    const int64_t step = kBackwardMaxBlocks * (info.backward_threads / kWaveSize)
+        * info.rows_per_wave / info.parts;
+    const int64_t steps = (c.rows + step - 1) / step;
+    const int64_t last = c.rows - (steps - 1) * step;
+    if (c.hidden > 2432) {
+        return c.hidden <= 6144
+            && (steps > 1 || (!c.has_grad_normalized && c.hidden <= 5120
+                              && c.rows * c.hidden <= (1 << 19)));
+    }
+    if (c.hidden > 2048) {
+        return steps == 2;
+    }
+    if (c.hidden > 1216) {
+        return (steps == 1 && 4 * last > 3 * step) || (steps == 2 && 2 * last > step);
+    }
+    return c.hidden <= 256 && !c.has_grad_normalized && steps == 1 && 3 * last > 2 * step;
 }
 
 inline bool single_backward(const SingleBackwardCall& c) {
@@ -232,7 +275,7 @@ inline bool single_backward(const SingleBackwardCall& c) {
         && backward_twelve_waves(c.hidden, c.rows)) {
         return false;
     }
-    return c.rows * c.hidden <= single_backward_most(c);
+    return c.rows * c.hidden <= single_backward_most(c) && (c.sums || !walk_without_sums(c));
 }
 
 // Rows of one chunk: its blocks run on one XCD, and its slab blocks read again
@@ -297,7 +340,8 @@ inline bool takes_single_backward(const BackwardArgs& a, int64_t hidden, int bra
                                   int grad_normalized_dtype, bool aligned) {
     const bool sums = (a.flags & kParameters) != 0;
     const bool partials = (a.flags & kPartials) != 0;
-    return single_backward({a.rows, hidden, grad_normalized_dtype, sums, partials, aligned})
+    return single_backward({a.rows, hidden, grad_normalized_dtype,
+                            (a.flags & kHasGradNormalized) != 0, sums, partials, aligned})
         && !(partials && !single_partials(a.rows, hidden))
         && !(sums && gradients_over_inputs(a, hidden, branch_dtype, grad_normalized_dtype));
 }

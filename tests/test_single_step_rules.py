@@ -74,6 +74,7 @@ def test_gradients_over_inputs_walk(ask, hidden):
 # (rows, hidden, branch, grad_normalized, flags, single-step?) on both sides of
 # lines beside which rln_single.h gives both sides' times.
 NONE = EVERYTHING & ~PARAMETERS
+NO_GRAD_NORMALIZED = NONE & ~GRAD_NORMALIZED
 MISALIGNED = [
     (5792, 128, F16, F32, EVERYTHING, 1), (11585, 128, F32, F32, EVERYTHING, 0),
     (5461, 768, F32, F32, EVERYTHING, 1), (6553, 640, BF16, BF16, EVERYTHING, 1),
@@ -108,3 +109,26 @@ def test_deterministic_route_ignores_alignment(ask):
     queries = [("backward", rows, hidden, F16, F32, EVERYTHING | PARTIALS, 0)
                for hidden in HIDDEN for rows in (1, 60, 300, 1000, 3000, 9000, 20000)]
     assert ask([(*q, 0) for q in queries]) == ask([(*q, 1) for q in queries])
+
+
+WITHOUT_SUMS = [
+    (241, 3072, F16, F32, NONE, 1), (482, 3072, F16, F32, NONE, 0), (512, 4096, F32, F32, NONE, 0),
+    (682, 6144, BF16, BF16, NONE, 0), (682, 6144, BF16, BF16, EVERYTHING, 1),
+    (42, 3072, F16, F32, NO_GRAD_NORMALIZED, 0), (42, 3072, F16, F32, NONE, 1),
+    (241, 3072, F16, F32, NO_GRAD_NORMALIZED, 1), (85, 6144, F16, F32, NO_GRAD_NORMALIZED, 1),
+    (512, 2048, F16, F32, NONE, 1), (579, 1280, F16, F32, NONE, 0), (655, 1600, F16, F32, NONE, 0),
+    (724, 2048, F32, F32, NONE, 0), (724, 2048, F32, F32, EVERYTHING, 1),
+    (926, 1600, F16, F32, NONE, 1), (1170, 1792, F32, F32, NONE, 0),
+    (431, 2432, F16, F32, NONE, 1), (862, 2432, F16, F32, NONE, 0),
+    (4096, 128, F16, F32, NO_GRAD_NORMALIZED, 0), (4096, 128, F16, F32, NONE, 1),
+    (5792, 128, F16, F32, NO_GRAD_NORMALIZED, 1),
+    (362, 8192, F16, F32, NONE, 1), (512, 8192, F32, F32, NONE, 0), (512, 8192, F32, F32, EVERYTHING, 1),
+    (1170, 7168, F16, F32, NONE, 1),
+]
+
+
+def test_backward_lines_without_sums(ask):
+    """Frozen parameters, or no grad_normalized: the walking backward where its
+    grid is full in its first or second row step."""
+    assert ask([("backward", *case[:5], 0, 1) for case in WITHOUT_SUMS]) \
+        == [[case[5]] for case in WITHOUT_SUMS]
