@@ -189,8 +189,19 @@ __device__ __forceinline__ void row_handoff(int parts) {
 // 49.7, [712, 4160] 29.6 -> 33.4, [675, 6208] fp32 51.1 -> 60.2, [682, 6144] fp32 42.5 ->
 // 63.1. Without sums, where only the row chains can gain: [204, 1280] 5.8 -> 4.7,
 // [579, 1280] 8.3 -> 9.6, and rows of 2433-6144 columns lose at every size ([21,
-// 3072] 4.4 -> 4.6, [482, 3072] 12.2 -> 14.8). Deterministic sums are the same bits
-// for tensors of any alignment, so their line does not ask for it.
+// 3072] 4.4 -> 4.6, [482, 3072] 12.2 -> 14.8).
+//
+// Deterministic launches put partials into the workspace instead of adding
+// atomics, so the row chains alone pay for the second read, up to 2 M elements
+// for 320-768 columns, 3 M up to 2432, 4 M, 6 M and 12 M for longer rows: [2730, 768]
+// 17.0 -> 13.6, [2048, 1024] 13.5 -> 12.0, [1310, 1600] 14.2 -> 13.2, [965, 3072] 19.3 ->
+// 16.3, [819, 5120] 26.6 -> 21.9, [827, 7168] 37.6 -> 29.4, [1448, 256] 9.6 -> 6.8; past the
+// lines [5461, 768] 19.9 -> 21.4, [13107, 640] 32.6 -> 36.1, [8192, 1024] 31.1 -> 33.1,
+// [3707, 1600] 24.8 -> 26.2, [1655, 3584] 27.4 -> 28.7, [1638, 5120] 35.6 -> 38.8, [2702,
+// 6208] 72.5 -> 75.9, [5792, 256] 11.1 -> 11.7, [1930, 192] bf16 6.8 -> 7.1, [4096, 128] 7.5 ->
+// 8.2. The sums are the same bits for tensors of any alignment, so these lines do
+// not ask for it (element accesses alone would walk from 1 M elements: [1310, 1600]
+// 21.1 -> 24.3).
 struct SingleBackwardCall {
     int64_t rows;
     int64_t hidden;
@@ -213,7 +224,17 @@ inline int64_t single_backward_most(const SingleBackwardCall& c) {
         {256, M, 256 * K},  {768, 12 * M, 12 * M}, {1024, M, 384 * K},           {2432, M, 512 * K},
         {4096, M, 0},       {6144, 1536 * K, 0},   {kMaxHidden, 3 * M, 2 * M},
     };
-    if (!c.aligned && !c.partials) {
+    if (c.partials) {
+        return c.hidden == 128  ? 384 * K
+            : c.hidden == 192   ? 256 * K
+            : c.hidden == 256   ? 768 * K
+            : c.hidden <= 768   ? 2 * M
+            : c.hidden <= 2432  ? 3 * M
+            : c.hidden < 4096   ? 4 * M
+            : c.hidden <= 6144  ? 6 * M
+                                : 12 * M;
+    }
+    if (!c.aligned) {
         for (const Misaligned& line : kMisaligned) {
             if (c.hidden <= line.hidden) {
                 return c.sums ? line.sums : line.none;
@@ -300,15 +321,6 @@ inline int64_t single_partial_rows(int64_t rows, int64_t hidden, const SingleSpl
     return least > chunk ? least : chunk;
 }
 
-// Past 64 rows per group of a full workspace, chunks fall out of L2 and the
-// walking backward is faster ([131072, 128] deterministic 57.5 against 64.8
-// us), and at 128 columns, where the row teams leave half their lanes idle
-// and nothing is gained on atomics, already from 4096 rows ([8192, 128] 9.1
-// against 11.1 us; [16384, 512] 30.7 -> 30.1 single-step).
-inline bool single_partials(int64_t rows, int64_t hidden) {
-    return rows <= (hidden == 128 ? 4096 : 64 * kBackwardMaxBlocks);
-}
-
 // Whether two device ranges share a byte (null: no range).
 inline bool ranges_overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
     const uintptr_t first = reinterpret_cast<uintptr_t>(a);
@@ -342,7 +354,6 @@ inline bool takes_single_backward(const BackwardArgs& a, int64_t hidden, int bra
     const bool partials = (a.flags & kPartials) != 0;
     return single_backward({a.rows, hidden, grad_normalized_dtype,
                             (a.flags & kHasGradNormalized) != 0, sums, partials, aligned})
-        && !(partials && !single_partials(a.rows, hidden))
         && !(sums && gradients_over_inputs(a, hidden, branch_dtype, grad_normalized_dtype));
 }
 

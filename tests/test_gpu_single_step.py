@@ -102,7 +102,10 @@ def test_single_step_rows_equal_walked_rows(hidden, dropout_p):
 
 @pytest.mark.parametrize("rows,hidden", [(3, 384), (300, 192), (4096, 128), (4097, 128),
                                          (9000, 256), (16384, 512), (16385, 512), (500, 2880),
-                                         (33, 8192)])
+                                         (33, 8192), (3072, 128), (3073, 128), (3072, 256),
+                                         (3073, 256), (4096, 512), (4097, 512), (3072, 1024),
+                                         (3073, 1024), (1365, 3072), (1366, 3072), (1228, 5120),
+                                         (1229, 5120), (1536, 8192), (1537, 8192)])
 def test_deterministic_partials(rows, hidden):
     """Fixed-order weight/bias sums of single-step launches: chunks of few and
     many rows, and the row counts that hand over to the walking backward. Bit

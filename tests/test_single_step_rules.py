@@ -132,3 +132,17 @@ def test_backward_lines_without_sums(ask):
     grid is full in its first or second row step."""
     assert ask([("backward", *case[:5], 0, 1) for case in WITHOUT_SUMS]) \
         == [[case[5]] for case in WITHOUT_SUMS]
+
+
+DETERMINISTIC = [
+    (2896, 128, 1), (4096, 128, 0), (1365, 192, 1), (1930, 192, 0), (1448, 256, 1), (5792, 256, 0),
+    (2730, 768, 1), (5461, 768, 0), (3276, 640, 1), (13107, 640, 0), (2048, 1024, 1), (8192, 1024, 0),
+    (1310, 1600, 1), (3707, 1600, 0), (965, 3072, 1), (1655, 3584, 0), (819, 5120, 1), (1638, 5120, 0),
+    (827, 7168, 1), (2702, 6208, 0),
+]
+
+
+def test_deterministic_backward_lines(ask):
+    """Fixed-order sums: the walking backward past the lines of their own."""
+    assert ask([("backward", rows, hidden, F16, F32, EVERYTHING | PARTIALS, 0, 1)
+                for rows, hidden, _ in DETERMINISTIC]) == [[case[2]] for case in DETERMINISTIC]
