@@ -199,7 +199,10 @@
 // [65536, 256] +2 to +4 %, [65536, 1024] +1.2 %, [16384, 4096] +1.5 %; and
 // past the lines [262144, 128] -1 %, [131072, 256] 0 %, [87381, 768] -0.8 %,
 // [174762, 768] -1.0 %, [131072, 1024] -0.6 to +0.3 %. (A large backward loses
-// 1-3 %.) The switch is the line of the shortest rows. Misaligned launches, whose
+// 1-3 %.) With dropout, rows of more than 4096 columns stop gaining at 2^25:
+// forward and backward [5405, 6208] 209.1 -> 207.7, [5792, 8192] 278.4 -> 284.9, [9362,
+// 7168] 390.5 -> 399.6; without it they gain up to 2^26 (forward [8192, 8192] 176.8 ->
+// 159.4). The switch is the line of the shortest rows. Misaligned launches, whose
 // element stores write through a part of a line at a time, keep the line of
 // RLN_WRITE_THROUGH_ELEMENTS ([7414, 1600] 96.2 non-temporal, 114.8 us write-through,
 // [10485, 1600] bf16 94.5 and 137.9, [65536, 256] 145.6 and 162.4).
@@ -860,11 +863,12 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // The descriptor's fourth word for a raw (untyped, unswizzled) buffer.
 constexpr int kRawBufferWord3 = 0x00020000;
-inline int forward_write_through(int64_t rows, int64_t hidden, bool aligned) {
+inline int forward_write_through(int64_t rows, int64_t hidden, bool dropout, bool aligned) {
     if (!aligned) {
         return rows * hidden < RLN_WRITE_THROUGH_ELEMENTS ? 1 : 0;
     }
-    const int64_t line = hidden >= 1024 ? 4 * RLN_FWD_WRITE_THROUGH_ELEMENTS
+    const int64_t line = hidden > 4096 && dropout ? 2 * RLN_FWD_WRITE_THROUGH_ELEMENTS
+        : hidden >= 1024                ? 4 * RLN_FWD_WRITE_THROUGH_ELEMENTS
         : hidden >= 512                 ? 2 * RLN_FWD_WRITE_THROUGH_ELEMENTS
                                         : RLN_FWD_WRITE_THROUGH_ELEMENTS;
     return rows * hidden <= line ? 1 : 0;
@@ -2181,7 +2185,7 @@ int launch_forward_walk(const ForwardArgs& a, S shape) {
         a.threshold,
         a.philox,
         forward_paced(a.rows, shape.hidden()),
-        forward_write_through(a.rows, shape.hidden(), Aligned));
+        forward_write_through(a.rows, shape.hidden(), a.dropout != 0, Aligned));
     return check_launch("rln_forward_kernel");
 }
 

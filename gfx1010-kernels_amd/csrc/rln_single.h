@@ -123,7 +123,9 @@ SingleSplit single_split(int64_t hidden, int64_t rows) {
 // [4139, 768] 11.9 -> 12.1; [4096, 512] 9.4 -> 7.1, [6208, 512] 11.3 -> 11.4;
 // [8192, 128] 7.0 -> 7.8; [655, 1600] 5.6 -> 5.1, [993, 1600] 6.2 -> 6.4).
 // Without dropout, rows above 4096 columns only for a few rows ([1, 8192]
-// 5.0 -> 4.7 us, [32, 8192] 5.3 -> 5.6; with dropout [128, 8192] 7.2 -> 6.7).
+// 5.0 -> 4.7 us, [32, 8192] 5.3 -> 5.6; with dropout [128, 8192] 7.2 -> 6.7), and
+// rows of 128 columns only up to one row step of the walk, 4096 rows ([4096,
+// 128] 4.3 -> 4.1, [5792, 128] 4.5 -> 4.9; with dropout [5792, 128] 6.8 -> 6.6).
 //
 // Misaligned tensors (element accesses) up to 384 K elements (512 K for 512-1024
 // columns) of rows of at most 4096 columns: from there four times the access
@@ -141,7 +143,8 @@ inline bool single_forward(int64_t rows, int64_t hidden, bool dropout, bool alig
     if (hidden > 4096 && !dropout) {
         return elements <= (1 << 17);
     }
-    return rows <= 6144 && elements <= (hidden <= 1280 ? 1 << 21 : 1 << 20);
+    return rows <= (hidden == 128 && !dropout ? 4096 : 6144)
+        && elements <= (hidden <= 1280 ? 1 << 21 : 1 << 20);
 }
 
 // Orders a block's LDS writes before its reads: a barrier where several waves
@@ -156,7 +159,8 @@ __device__ __forceinline__ void row_handoff(int parts) {
 }
 
 // The backward runs single-step up to 12 M elements (2^24 above 6144 columns,
-// 2^23 for 256 and 4096-6144, 6 M for 1025-4095, 2^22 for 128), where the
+// 2^23 for 256 and 4096-6144, 6 M for 1025-3072, 4 M there with a 32-bit branch
+// and gradient, 3 M for 3073-4095, 2^22 for 128), where the
 // walking backward's own costs - the fixed part of its row chains, and the
 // weight/bias atomics of its up to 256 blocks, which grow with the row length
 // and not with the rows - outweigh reading `updated` and grad_normalized a
@@ -170,7 +174,9 @@ __device__ __forceinline__ void row_handoff(int parts) {
 // 32.1 -> 31.5, [61445, 128] fp16 out 47.2 -> 48.5, [32768, 256] 53.2 -> 50.6,
 // [52119, 256] fp32 branch 84.2 -> 85.0, [16555, 768] 77.4 -> 75.7, [21845, 768]
 // 95.8 -> 96.9, [3973, 1600] 45.0 -> 43.6, [2207, 2880] 45.2 -> 45.9, [2048,
-// 4096] 55.4 -> 55.4, [2048, 8192] 116.6 -> 110.9.
+// 4096] 55.4 -> 55.4, [2048, 8192] 116.6 -> 110.9; with a 32-bit branch and gradient,
+// backward alone, [2621, 1600] 18.6 -> 18.5, [3707, 1600] 23.4 -> 25.0; [827, 3584] 18.8 -> 16.0,
+// [1170, 3584] 20.1 -> 21.4, [1655, 3584] fp16 23.8 -> 25.3.
 //
 // Not where the walking backward runs its staggered twelve-wave blocks over
 // three row steps (768 columns, 7168 rows and more) with a 32-bit
@@ -205,6 +211,7 @@ __device__ __forceinline__ void row_handoff(int parts) {
 struct SingleBackwardCall {
     int64_t rows;
     int64_t hidden;
+    int branch_dtype;
     int grad_normalized_dtype;
     bool has_grad_normalized;
     bool sums;      // weight and bias sums, by atomics or ...
@@ -241,13 +248,17 @@ inline int64_t single_backward_most(const SingleBackwardCall& c) {
             }
         }
     }
-    return c.hidden == 128   ? 4 * M
-        : c.hidden == 256    ? 8 * M
-        : c.hidden <= 1024   ? 12 * M
-        : c.hidden < 4096    ? 6 * M
-        : c.hidden <= 6144   ? 8 * M
+    const bool wide =
+        c.branch_dtype == RLN_DTYPE_F32 && c.grad_normalized_dtype == RLN_DTYPE_F32;
+    return c.hidden == 128           ? 4 * M
+        : c.hidden == 256            ? 8 * M
+        : c.hidden <= 1024           ? 12 * M
+        : c.hidden <= 3072           ? (wide ? 4 * M : 6 * M)
+        : c.hidden < 4096            ? 3 * M
+        : c.hidden <= 6144           ? 8 * M
         : c.hidden <= 7936 || c.sums ? 16 * M
-                                     : 3 * M;
+        : wide                       ? 3 * M
+                                     : 5 * M;
 }
 
 // A backward without weight/bias sums (frozen parameters, or no grad_normalized)
@@ -268,9 +279,9 @@ inline int64_t single_backward_most(const SingleBackwardCall& c) {
 //    backward [609, 2432] 16.3 -> 17.4);
 //  * rows of 128-256 columns without grad_normalized in the first step: [4096, 128]
 //    3.7 -> 4.0, [5792, 128] 5.3 -> 4.5;
-//  * rows of 8000-8192 columns lose from 3 M elements ([362, 8192] 18.1 -> 13.7, [512,
-//    8192] fp32 22.1 -> 25.0, [1448, 8192] 45.5 -> 50.8), shorter ones up to 7936 do not
-//    ([1170, 7168] 33.5 -> 34.3).
+//  * rows of 8000-8192 columns lose from 5 M elements, 3 M with a 32-bit branch and
+//    gradient ([362, 8192] 18.1 -> 13.7, [512, 8192] 21.6 -> 18.2, fp32 22.1 -> 25.0, [1448,
+//    8192] 45.5 -> 50.8), shorter ones up to 7936 do not ([1170, 7168] 33.5 -> 34.3).
 inline bool walk_without_sums(const SingleBackwardCall& c) {
     const ShapeInfo info = shape_info(c.hidden, Pass::kBackward, c.rows);
     const int64_t step = kBackwardMaxBlocks * (info.backward_threads / kWaveSize)
@@ -352,7 +363,7 @@ inline bool takes_single_backward(const BackwardArgs& a, int64_t hidden, int bra
                                   int grad_normalized_dtype, bool aligned) {
     const bool sums = (a.flags & kParameters) != 0;
     const bool partials = (a.flags & kPartials) != 0;
-    return single_backward({a.rows, hidden, grad_normalized_dtype,
+    return single_backward({a.rows, hidden, branch_dtype, grad_normalized_dtype,
                             (a.flags & kHasGradNormalized) != 0, sums, partials, aligned})
         && !(sums && gradients_over_inputs(a, hidden, branch_dtype, grad_normalized_dtype));
 }

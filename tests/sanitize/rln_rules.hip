@@ -78,7 +78,7 @@ int main() {
             bool dropout = false, aligned = true;
             in >> rows >> hidden >> dropout >> aligned;
             std::printf("%d %d\n", rln::single_forward(rows, hidden, dropout, aligned),
-                        rln::forward_write_through(rows, hidden, aligned));
+                        rln::forward_write_through(rows, hidden, dropout, aligned));
         } else {
             query.clear();
         }

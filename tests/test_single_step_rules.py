@@ -146,3 +146,22 @@ def test_deterministic_backward_lines(ask):
     """Fixed-order sums: the walking backward past the lines of their own."""
     assert ask([("backward", rows, hidden, F16, F32, EVERYTHING | PARTIALS, 0, 1)
                 for rows, hidden, _ in DETERMINISTIC]) == [[case[2]] for case in DETERMINISTIC]
+
+
+def test_lines_of_32_bit_tensors_and_long_rows(ask):
+    """A 32-bit branch and gradient pass over to the walk earlier, and so do rows of
+    3073-4095 columns."""
+    cases = [(2621, 1600, F32, F32, EVERYTHING, 1), (3707, 1600, F32, F32, EVERYTHING, 0),
+             (3707, 1600, F16, F32, EVERYTHING, 1), (3707, 1600, F32, F32, NONE, 0),
+             (827, 3584, F32, F32, EVERYTHING, 1), (1170, 3584, F32, F32, EVERYTHING, 0),
+             (1655, 3584, F16, F32, EVERYTHING, 0), (512, 8192, F16, F32, NONE, 1),
+             (1448, 8192, F16, F32, NONE, 0)]
+    assert ask([("backward", *case[:5], 0, 1) for case in cases]) == [[case[5]] for case in cases]
+
+
+def test_forward_lines(ask):
+    """Aligned forwards: (rows, hidden, dropout) single-step and write-through."""
+    cases = [(4096, 128, 0, 1, 1), (5792, 128, 0, 0, 1), (5792, 128, 1, 1, 1), (5792, 256, 0, 1, 1),
+             (5405, 6208, 1, 0, 1), (5792, 8192, 1, 0, 0), (9362, 7168, 1, 0, 0),
+             (8192, 8192, 0, 0, 1), (8193, 8192, 0, 0, 0), (16384, 4096, 1, 0, 1)]
+    assert ask([("forward", *case[:3], 1) for case in cases]) == [list(case[3:]) for case in cases]
