@@ -10,9 +10,10 @@
 // several rows one after the other on a few of the 256 CUs, behind unrolled
 // walks and, with dropout, a Philox chain of 2-4 draws per lane. Here
 //  * a row is split over more waves, one to four four-element slots per lane,
-//    so a lane holds 36-90 VGPRs, 5-8 waves fit a SIMD, and rows spread over
-//    every CU; row sums cross the waves in LDS, in the walking shape's order,
-//    so both kernels give a row the same bits;
+//    so a lane holds 36-96 VGPRs (forward) or 57-90 (backward) over all types and
+//    alignments, 5-8 waves fit a SIMD, and rows spread over every CU; row sums
+//    cross the waves in LDS, in the walking shape's order, so both kernels give a
+//    row the same bits;
 //  * no loop: one row's loads, sums and stores are the whole kernel;
 //  * rows are read through buffer descriptors over exactly the row, so lanes
 //    past its end read zeros and store nothing, without a branch;
@@ -27,6 +28,22 @@
 #define RLN_SINGLE_H
 
 #include "rln_device.h"
+
+// Switches for A/B builds (bench.py --ab): 0 keeps a pass on the walking kernels
+// at every size; 1 gives 768 columns with 32-bit gradients the line of the others
+// (single_backward_most); and the rows of a chunk (single_chunk_rows), 0 = by rule.
+#ifndef RLN_FWD_SINGLE_STEP
+#define RLN_FWD_SINGLE_STEP 1
+#endif
+#ifndef RLN_BWD_SINGLE_STEP
+#define RLN_BWD_SINGLE_STEP 1
+#endif
+#ifndef RLN_BWD_SINGLE_STEP_768
+#define RLN_BWD_SINGLE_STEP_768 0
+#endif
+#ifndef RLN_SINGLE_CHUNK_ROWS
+#define RLN_SINGLE_CHUNK_ROWS 0
+#endif
 
 namespace rln {
 
@@ -136,6 +153,9 @@ SingleSplit single_split(int64_t hidden, int64_t rows) {
 // 8192] with it 9.4 -> 10.3).
 inline bool single_forward(int64_t rows, int64_t hidden, bool dropout, bool aligned) {
     const int64_t elements = rows * hidden;
+    if (!RLN_FWD_SINGLE_STEP) {
+        return false;
+    }
     if (!aligned) {
         return hidden <= 4096
             && elements <= (hidden >= 512 && hidden <= 1024 ? 512 << 10 : 384 << 10);
@@ -178,13 +198,21 @@ __device__ __forceinline__ void row_handoff(int parts) {
 // backward alone, [2621, 1600] 18.6 -> 18.5, [3707, 1600] 23.4 -> 25.0; [827, 3584] 18.8 -> 16.0,
 // [1170, 3584] 20.1 -> 21.4, [1655, 3584] fp16 23.8 -> 25.3.
 //
-// Not where the walking backward runs its staggered twelve-wave blocks over
-// three row steps (768 columns, 7168 rows and more) with a 32-bit
-// grad_normalized: alone single-step is faster there too ([8192, 768] 24.2 ->
-// 21.6 us), but a forward right after it takes 1.9 us longer when the batches
-// that alternate fit the 256 MB Infinity Cache by half (forward + backward
-// over three batches 39.9 against 41.6 us, over eight 41.9 against 40.1; with
-// 16-bit gradients 39.2 -> 37.0 over three).
+// Rows of 768 columns with a 32-bit grad_normalized and weight/bias sums pass over
+// to the walk at 7168 rows already: from there single-step is still faster alone
+// ([8192, 768] 23.1 -> 20.2), but a forward right after it takes 1-3 us longer as long
+// as the batches that alternate are few enough to stay partly in the 256 MB
+// Infinity Cache. Forward and backward, fp16 branch, walking -> single-step, over
+// three / four / eight batches: 6656 rows 35.6 -> 34.0 / 36.0 -> 34.8 / 38.5 -> 35.9;
+// 7168 35.6 -> 36.4 / 35.9 -> 36.9 / 38.1 -> 37.1; 7936 38.9 -> 40.4 / 39.5 -> 40.2 /
+// 41.6 -> 40.4; 8192 39.3 -> 40.7 / 39.5 -> 41.2 / 41.8 -> 40.9; 9217 44.6 -> 45.5 /
+// 45.3 -> 46.4 / 46.5 -> 46.3; 11264 52.3 -> 52.3 / 52.2 -> 52.6 / 54.0 -> 52.6; 13312
+// 59.0 -> 60.4 / 58.8 -> 60.5 / 61.5 -> 60.5; 15360 67.7 -> 68.9 / 67.2 -> 68.8 / 70.0 ->
+// 68.9 (fp32 branch: the same signs). So the walk is the choice for programs of a few
+// layers, and costs those with many between a forward and its backward 1-3 %.
+// Nothing of it shows with 16-bit gradients ([8192, 768] 37.9 -> 36.1 over three), at 640
+// and 896 columns (5120-16384 rows, three batches: 0.88-1.01 and 0.91-1.00 of the walk)
+// or without the sums.
 //
 // Misaligned tensors (element accesses) have lines of their own. At 320-768
 // columns, whose rows hold one slot per lane, they are the same ([5461, 768] 33.7
@@ -252,6 +280,9 @@ inline int64_t single_backward_most(const SingleBackwardCall& c) {
         c.branch_dtype == RLN_DTYPE_F32 && c.grad_normalized_dtype == RLN_DTYPE_F32;
     return c.hidden == 128           ? 4 * M
         : c.hidden == 256            ? 8 * M
+        : c.hidden == 768 && c.sums && c.grad_normalized_dtype == RLN_DTYPE_F32
+                && !RLN_BWD_SINGLE_STEP_768
+            ? 7167 * 768
         : c.hidden <= 1024           ? 12 * M
         : c.hidden <= 3072           ? (wide ? 4 * M : 6 * M)
         : c.hidden < 4096            ? 3 * M
@@ -303,22 +334,27 @@ inline bool walk_without_sums(const SingleBackwardCall& c) {
 }
 
 inline bool single_backward(const SingleBackwardCall& c) {
-    if (c.grad_normalized_dtype == RLN_DTYPE_F32 && c.rows >= 7168
-        && backward_twelve_waves(c.hidden, c.rows)) {
+    if (!RLN_BWD_SINGLE_STEP) {
         return false;
     }
     return c.rows * c.hidden <= single_backward_most(c) && (c.sums || !walk_without_sums(c));
 }
 
 // Rows of one chunk: its blocks run on one XCD, and its slab blocks read again
-// from that XCD's L2 what its row blocks read. 64 rows (32 where a block has
-// three waves: whole steps of the slab blocks), fewer when there are fewer
-// rows than eight such chunks, one per XCD, so that every XCD has work.
-// Smaller chunks mean more weight/bias atomics, larger ones fall out of L2:
-// [8192, 768] 21.9 us at 32 rows, 22.7 at 64, 23.5 at 128; [8192, 1600] 44.5, 43.2,
-// 43.8; [16384, 128] 16.3, 10.4, 10.6.
+// from that XCD's L2 what its row blocks read. 64 rows, 32 where a block has
+// three waves (513-768 columns: its slab has three quarters of the waves of the
+// others', and takes as long for fewer rows), fewer when there are fewer rows than
+// eight such chunks, one per XCD, so that every XCD has work. Smaller chunks mean
+// more weight/bias atomics, larger ones longer slab blocks, and past L2's size a
+// second read from memory: [8192, 768] 21.9 us at 32 rows, 22.7 at 64, 23.5 at 128;
+// [8192, 1600] 44.5, 43.2, 43.8; [16384, 128] 16.3, 10.4, 10.6. At 513-768 columns over
+// 2^17-2^23 elements, against 32 rows: 64 rows +1 to +14 %, 48 rows (a whole
+// unrolled step of three waves) -2 to +2 % but +3 to +10 % at the rows that then leave
+// an XCD idle ([482, 768]).
 inline int64_t single_chunk_rows(int64_t rows, const SingleSplit& split) {
-    const int64_t most = split.waves() == 3 ? 32 : 64;
+    const int64_t most = RLN_SINGLE_CHUNK_ROWS ? RLN_SINGLE_CHUNK_ROWS
+        : split.waves() == 3                    ? 32
+                                                : 64;
     const int64_t spread = (rows + 7) / 8;
     return spread < most ? (spread + 3) / 4 * 4 : most;
 }

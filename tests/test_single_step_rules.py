@@ -165,3 +165,16 @@ def test_forward_lines(ask):
              (5405, 6208, 1, 0, 1), (5792, 8192, 1, 0, 0), (9362, 7168, 1, 0, 0),
              (8192, 8192, 0, 0, 1), (8193, 8192, 0, 0, 0), (16384, 4096, 1, 0, 1)]
     assert ask([("forward", *case[:3], 1) for case in cases]) == [list(case[3:]) for case in cases]
+
+
+def test_768_columns_with_32_bit_gradients_walk_from_7168_rows(ask):
+    """One line, whatever shape the walk has above it; 16-bit gradients, launches
+    without sums and the neighbouring row lengths keep theirs."""
+    rows = (6912, 7167, 7168, 7679, 7680, 8192, 9216, 9217, 16384)
+    for branch in (F16, F32):
+        assert ask([("backward", r, 768, branch, F32, EVERYTHING, 0, 1) for r in rows]) \
+            == [[int(r < 7168)] for r in rows]
+    for hidden, grad_normalized, flags in ((768, BF16, EVERYTHING), (768, F32, NONE),
+                                           (704, F32, EVERYTHING), (832, F32, EVERYTHING)):
+        assert ask([("backward", r, hidden, F16, grad_normalized, flags, 0, 1) for r in rows]) \
+            == [[int(r * hidden <= 12 << 20)] for r in rows]
