@@ -169,11 +169,11 @@
 // Cache policies of the row outputs' stores (every output the kernels write
 // per row: updated, normalized, the mask, mean and rstd, grad_x,
 // grad_branch), as the cache-policy bits of a gfx950 buffer store: sc0 = 1,
-// nt = 2, sc1 = 16. Launches over fewer than RLN_WRITE_THROUGH_ELEMENTS
-// elements write through the caches at system scope (sc0 | sc1), so that no
-// dirty line is left in L2 for the end-of-kernel release to write back;
-// larger launches store non-temporally (the forward from the larger sizes
-// below). Measured on MI355X (bench.py --ab, alternated): C1 [8192, 768] step
+// nt = 2, sc1 = 16. Backward launches over fewer than RLN_WRITE_THROUGH_ELEMENTS
+// elements (the forward up to the larger lines below) write through the caches at
+// system scope (sc0 | sc1), so that no dirty line is left in L2 for the
+// end-of-kernel release to write back; larger launches store non-temporally.
+// Measured on MI355X (bench.py --ab, alternated): C1 [8192, 768] step
 // 39.1 us write-through against 40.3 us non-temporal (forward 14.8 against
 // 17.0 us); at 2^26+ elements both passes write-through lose 1-7 % (C3 358.7
 // against 371.6 us, [262144, 384] 541 against 555 us). The
@@ -188,10 +188,11 @@
 #ifndef RLN_WRITE_THROUGH_ELEMENTS
 #define RLN_WRITE_THROUGH_ELEMENTS (1ll << 23)
 #endif
-// The forward writes through up to larger launches: 2^24 elements, 2^25 for
-// rows of 512 columns and more, 2^26 for 1024 and more. Its outputs are then in the Infinity Cache, not
-// in L2 lines still to be written back, when the kernel ends: it ends sooner and
-// a backward that follows reads them faster. Measured (us, non-temporal ->
+// The forward writes through up to larger launches: RLN_FWD_WRITE_THROUGH_ELEMENTS,
+// and twice that for rows of 512 columns and more, four times for 1024 and more
+// (forward_write_through). No L2 line is then left to be written back when the
+// kernel ends, and up to the 256 MB Infinity Cache (2^24 to 2^25 elements of outputs)
+// a backward that follows finds its inputs there. Measured (us, non-temporal ->
 // write-through): forward without dropout [6001, 2880] bf16 40.5 -> 38.7,
 // [32768, 1024] 81.3 -> 75.7, [8192, 4096] 85.2 -> 78.1; forward and backward
 // of the same batch [46340, 256] 69.6 -> 65.8, [43690, 768] 184.6 -> 178.1,
@@ -202,7 +203,7 @@
 // 1-3 %.) With dropout, rows of more than 4096 columns stop gaining at 2^25:
 // forward and backward [5405, 6208] 209.1 -> 207.7, [5792, 8192] 278.4 -> 284.9, [9362,
 // 7168] 390.5 -> 399.6; without it they gain up to 2^26 (forward [8192, 8192] 176.8 ->
-// 159.4). The switch is the line of the shortest rows. Misaligned launches, whose
+// 159.4). Misaligned launches, whose
 // element stores write through a part of a line at a time, keep the line of
 // RLN_WRITE_THROUGH_ELEMENTS ([7414, 1600] 96.2 non-temporal, 114.8 us write-through,
 // [10485, 1600] bf16 94.5 and 137.9, [65536, 256] 145.6 and 162.4).
@@ -455,7 +456,14 @@ inline bool backward_runs_wide(int64_t hidden, int64_t rows) {
 // 32.6, 8192 40.0 -> 39.2 (C1; bf16 output 38.2 -> 36.8); and slower at 4096
 // (26.0 -> 26.7) and 7168 (34.3 -> 35.8), where a third of the waves is busy
 // in the last step, equal at 10240 and 12288, 1-3 % slower from 16384 rows.
-// RLN_BWD_TWELVE_WAVE_768=0 keeps the eight-wave ring everywhere.
+// RLN_BWD_TWELVE_WAVE_768=0 keeps the eight-wave ring everywhere. Of these
+// launches the walk now gets (takes_single_backward in rln_single.h; the figures
+// above are the walk's, with weight/bias atomics, which builds with
+// RLN_BWD_SINGLE_STEP=0 measure again): 7680-9216 rows with a 32-bit
+// grad_normalized, deterministic ones from 2 M elements (2731 rows), and those whose
+// gradients are written over their inputs. Deterministic (no atomics, so less for
+// the stagger to gain), eight-wave ring -> twelve-wave walk: 5461 rows 20.0 -> 19.6, 8192
+// 24.6 -> 25.5, 9216 28.0 -> 27.3.
 #ifndef RLN_BWD_TWELVE_WAVE_768
 #define RLN_BWD_TWELVE_WAVE_768 1
 #endif
@@ -478,7 +486,11 @@ inline bool backward_twelve_waves(int64_t hidden, int64_t rows) {
 // 20.80 -> 20.00 at p = 0.1; fp16 branch 11520 rows 18.93 -> 18.63, 12291
 // 20.28 -> 19.13, 13000 21.79 -> 20.11. With the third step (nearly) full
 // the blocks end together and the copy walk only costs: 13823 rows 20.68 ->
-// 21.46, 13824 20.70 -> 21.43; with two steps, 7168 rows 13.58 -> 14.11.
+// 21.46, 13824 20.70 -> 21.43; with two steps, 7168 rows 13.58 -> 14.11. (The
+// commands need RLN_BWD_SINGLE_STEP=0 in both builds.) Atomic launches of this size
+// run single-step; deterministic ones walk (eight -> nine waves: 11520 rows 20.7 ->
+// 21.3, 12291 21.5 -> 21.6, 13000 23.5 -> 22.0), and so do gradients written over
+// their inputs.
 #ifndef RLN_BWD_NINE_WAVE_384
 #define RLN_BWD_NINE_WAVE_384 1
 #endif
@@ -502,7 +514,13 @@ inline bool backward_nine_waves(int64_t hidden, int64_t rows) {
 // 8192 27.74 -> 24.56; 2048 columns 4096 rows 30.20 -> 29.58, 8192 52.07 ->
 // 52.65. Larger launches lose (1024 columns: 12288 rows +0.7 %, 16384
 // +1.6 %; [262144, 1600] +5.7 %), and so do rows of three slots (2432
-// columns, 4096 rows 35.4 -> 41.9 us).
+// columns, 4096 rows 35.4 -> 41.9 us). (These commands, too, need
+// RLN_BWD_SINGLE_STEP=0 in both builds below 12 M elements at 769-1024 columns and 6 M
+// at 1217-2048.) The walk gets the launches above those sizes, deterministic ones
+// from 3 M elements, full grids without weight/bias sums at 1217-2048 columns
+// (walk_without_sums), and gradients written over their inputs. Deterministic, eight ->
+// twelve waves: [8192, 832] 28.2 -> 26.3, [4096, 1024] 19.2 -> 19.2, [2731, 1600] 21.2 ->
+// 20.6, [4096, 1600] 26.1 -> 26.6, [4096, 2048] 31.8 -> 33.0.
 #ifndef RLN_BWD_STAGGERED_WIDE
 #define RLN_BWD_STAGGERED_WIDE 1
 #endif

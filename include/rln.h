@@ -145,13 +145,18 @@ int rln_forward(
  * accumulate_parameters != 0 adds the parameter gradients to the values
  * already in grad_weight / grad_bias (gradient accumulation across calls, one
  * kernel launch in atomic mode); 0 overwrites them.
- * Placement (speed only): in atomic mode every block of the launch adds into
- * both arrays at its end. Measured at hidden = 768 (MI355X): when grad_bias
- * starts within 2 KiB of a multiple of 32 KiB after grad_weight (and at some
- * larger distances: 256 and 384 KiB, 4 MiB), both arrays fall on the same
- * memory channels and those atomics take about 3.7 times as long (6.2 instead
- * of 1.7 us per backward at [8192, 768]); adjacent arrays (two consecutive
- * allocations of `hidden` floats, or one [2, hidden] buffer) are fast.
+ * In atomic mode the launch adds partial sums into both arrays with fp32 atomics:
+ * once per chunk of 32-64 rows and column throughout a single-step launch (most
+ * launches below 4-16 million elements), once per block and column at the end of
+ * a larger one.
+ * Placement (speed only): measured at hidden = 768 on the larger kind (MI355X,
+ * [8192, 768] with fp32 gradients): when grad_bias starts within 2 KiB of a
+ * multiple of 32 KiB after grad_weight (and at some larger distances: 256 and 384
+ * KiB, 4 MiB), both arrays fall on the same memory channels and those atomics take
+ * about 3.7 times as long (6.2 instead of 1.7 us per backward); adjacent arrays
+ * (two consecutive allocations of `hidden` floats, or one [2, hidden] buffer) are
+ * fast. Single-step launches hardly depend on it ([1024, 384] 3.8 against 4.0 us;
+ * [4096, 768], [2048, 1600] and [8192, 768] with 16-bit gradients not at all).
  * workspace: device scratch of at least
  * rln_backward_workspace_bytes(rows, hidden, deterministic) bytes, 16-byte
  * aligned (may be NULL when that size is 0).
