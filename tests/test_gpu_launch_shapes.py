@@ -256,14 +256,18 @@ def test_sixteen_wave_backward_deterministic_and_half_gradient():
     check_parameter_gradients(outputs[0], grads[1], runs[0])
 
 
+# The walking backward's block shapes. Launches of many of these sizes run the
+# single-step backward (rln_single.h); _check_staggered_backward runs them in
+# place too, which always walks.
+#
 # Row counts of 768 columns around backward_twelve_waves (rln_device.h): the
-# backward runs twelve-wave blocks on the copy walk for 2048-9216 rows whose
+# walking backward runs twelve-wave blocks on the copy walk for 2048-9216 rows whose
 # last row step keeps at least half of the 256 x 12 waves busy (or all of
 # them), and the eight-wave ring otherwise.
 TWELVE_WAVE_CASES = [(2047, False), (2048, True), (4096, False), (5120, True), (7168, False),
                      (8192, True), (9216, True), (9217, False)]
 
-# Row counts of 384 columns around backward_nine_waves: nine-wave blocks of
+# Row counts of 384 columns around backward_nine_waves: nine-wave walking blocks of
 # two-row teams for 11520-13056 rows, eight-wave blocks otherwise; 12291 is
 # the C4 tail.
 NINE_WAVE_CASES = [(11519, False), (11520, True), (12291, True), (13056, True), (13057, False)]
@@ -271,7 +275,9 @@ NINE_WAVE_CASES = [(11519, False), (11520, True), (12291, True), (13056, True), 
 
 def _check_staggered_backward(rows, hidden, branch_dtype, mask_threads=128):
     """Whole tensors of the backward against the oracle; deterministic mode
-    replays bitwise, and its input gradients equal the atomic mode's.
+    replays bitwise, and its input gradients equal the atomic mode's. In place
+    (grad_x over grad_normalized: the walking shape itself) both modes give the
+    same input gradients, bit for bit, and sums at the parity bar.
     `mask_threads`: the dropout layout the forward draws (0 at the hidden
     sizes that only have the library's own)."""
     from test_gpu_backward import deterministic_algorithms
@@ -298,13 +304,41 @@ def _check_staggered_backward(rows, hidden, branch_dtype, mask_threads=128):
     assert torch.equal(first[0], atomic[0]) and torch.equal(first[1], atomic[1])
     check_parameter_gradients(outputs[0], grads[1], first)
 
+    walked = [_walked_backward(inputs[2], outputs, grads, branch_dtype, deterministic)
+              for deterministic in (False, True, True)]
+    for result in walked:
+        assert torch.equal(result[0], atomic[0]) and torch.equal(result[1], atomic[1])
+        check_parameter_gradients(outputs[0], grads[1], result)
+    assert torch.equal(walked[1][2], walked[2][2]) and torch.equal(walked[1][3], walked[2][3])
+
+
+def _walked_backward(weight, outputs, grads, branch_dtype, deterministic):
+    """The walking backward at any size: grad_x written over (a copy of)
+    grad_normalized, through the C ABI."""
+    code = {torch.float32: _cabi.RLN_DTYPE_F32, torch.float16: _cabi.RLN_DTYPE_F16,
+            torch.bfloat16: _cabi.RLN_DTYPE_BF16}
+    updated, _, mean, rstd, mask = outputs
+    rows, hidden = updated.numel() // updated.shape[-1], updated.shape[-1]
+    grad_x = grads[1].clone()
+    grad_branch = torch.empty_like(updated, dtype=branch_dtype)
+    grad_weight, grad_bias = torch.empty(2, hidden, device="cuda")
+    workspace = torch.empty(_cabi.backward_workspace_bytes(rows, hidden, deterministic),
+                            dtype=torch.uint8, device="cuda")
+    _cabi.backward(grads[0].data_ptr(), grad_x.data_ptr(), updated.data_ptr(), weight.data_ptr(),
+                   mean.data_ptr(), rstd.data_ptr(), mask.data_ptr(), grad_x.data_ptr(),
+                   grad_branch.data_ptr(), code[branch_dtype], grad_weight.data_ptr(),
+                   grad_bias.data_ptr(), rows, hidden, 0.1, True, deterministic,
+                   workspace.data_ptr() if deterministic else None, workspace.numel(),
+                   torch.cuda.current_stream().cuda_stream)
+    return grad_x, grad_branch, grad_weight, grad_bias
+
 
 @pytest.mark.parametrize("rows,twelve_waves", TWELVE_WAVE_CASES,
                          ids=[f"{rows}-{'twelve' if twelve else 'eight'}"
                               for rows, twelve in TWELVE_WAVE_CASES])
 def test_backward_twelve_wave_switch(rows, twelve_waves):
-    """Both sides of the switch between eight- and twelve-wave backward blocks
-    at 768 columns."""
+    """Both sides of the switch between eight- and twelve-wave walking backward
+    blocks at 768 columns."""
     hidden = 768
     teams = 256 * 12
     last = rows % teams
@@ -317,7 +351,7 @@ def test_backward_twelve_wave_switch(rows, twelve_waves):
                          ids=[f"{rows}-{'nine' if nine else 'eight'}"
                               for rows, nine in NINE_WAVE_CASES])
 def test_backward_nine_wave_switch(rows, nine_waves):
-    """Both sides of the switch between eight- and nine-wave backward blocks
+    """Both sides of the switch between eight- and nine-wave walking backward blocks
     at 384 columns, with the C4 tail's fp32 branch."""
     hidden = 384
     slots = 256 * 9 * 2
@@ -327,7 +361,7 @@ def test_backward_nine_wave_switch(rows, nine_waves):
 
 
 # Four-wave rows of one or two slots per lane (769-1024 and 1217-2048
-# columns) run their backward in twelve-wave blocks (StaggeredWideShape) up
+# columns) walk their backward in twelve-wave blocks (StaggeredWideShape) up
 # to 8192 rows; rows of three slots (2049-2432 columns) and of two waves
 # (1025-1216) keep eight-wave blocks.
 STAGGERED_WIDE_CASES = [(1600, 100, True), (1600, 8192, True), (1600, 8193, False),
@@ -355,7 +389,7 @@ def test_backward_staggered_wide_switch(hidden, rows, staggered):
 
 # One launch of each staggered backward shape (TwelveWaveShape<768>,
 # NineWaveShape<384>, StaggeredWideShape<2> and <1>), with the branch type
-# each serves in the sweep.
+# each serves in the sweep; deterministic launches of these sizes walk.
 STAGGERED_SHAPES = [(768, 8192, torch.float16), (384, 12291, torch.float32),
                     (1600, 4096, torch.float16), (1024, 4096, torch.float16)]
 

@@ -1,4 +1,4 @@
-"""Both row schedules of the kernels give the same bits.
+"""Both row schedules of the walking kernels give the same bits.
 
 The library walks a launch's rows with one row of look-ahead when it is
 small and paced (each row's loads issued after the previous row is stored,
@@ -10,7 +10,9 @@ a paced launch must equal, bit for bit, a look-ahead launch over just those
 rows; every row of the paced launch is also checked against the oracle
 (parity.check_full_tensor: the whole mask, `updated` bitwise, the rest
 against float64), its sums against a float64 reduction, and the
-element-access (misaligned) path against the aligned one. Calls go through
+element-access (misaligned) path against the aligned one. Most of these
+backwards would run single-step; they write grad_x over grad_normalized, which
+keeps them on the walk. Calls go through
 the C ABI with explicit Philox seeds and offsets (the library's own dropout
 layout).
 """
@@ -50,8 +52,10 @@ def make_case(rows, hidden, branch_dtype):
             randn(rows, hidden))
 
 
-def run(case, rows, normalized_dtype, dropout_p, deterministic, shift=0):
-    """Forward then backward over the first `rows` rows of `case`."""
+def run(case, rows, normalized_dtype, dropout_p, deterministic, shift=0, walk=False):
+    """Forward then backward over the first `rows` rows of `case`. `walk`: grad_x is
+    written over grad_normalized (a copy, fp32), which takes the walking backward at
+    every size (takes_single_backward in rln_single.h)."""
     x, branch, weight, bias, grad_updated, grad_normalized = case
     hidden = x.shape[1]
     stream = torch.cuda.current_stream().cuda_stream
@@ -70,6 +74,9 @@ def run(case, rows, normalized_dtype, dropout_p, deterministic, shift=0):
                   out["mean"].data_ptr(), out["rstd"].data_ptr(), out["mask"].data_ptr(),
                   rows, hidden, dropout_p, EPS, True, _cabi.RlnPhilox(SEED, OFFSET, None, None),
                   stream, normalized_dtype=CODE[normalized_dtype])
+    if walk:
+        out["grad_x"].copy_(grad_normalized[:rows])
+        grad_normalized = out["grad_x"]
     workspace = None
     if deterministic:
         size = _cabi.backward_workspace_bytes(rows, hidden, True)
@@ -123,8 +130,8 @@ def test_paced_rows_equal_look_ahead_rows(hidden, branch_dtype, normalized_dtype
     print(f"[schedules] H={hidden} rows={paced_rows}/{prefix} {branch_dtype} {normalized_dtype}",
           flush=True)
     case = make_case(paced_rows, hidden, branch_dtype)
-    paced = run(case, paced_rows, normalized_dtype, 0.1, deterministic=False)
-    look_ahead = run(case, prefix, normalized_dtype, 0.1, deterministic=False)
+    paced = run(case, paced_rows, normalized_dtype, 0.1, deterministic=False, walk=True)
+    look_ahead = run(case, prefix, normalized_dtype, 0.1, deterministic=False, walk=True)
     for name in ROW_OUTPUTS:
         assert_same_bits(paced[name][:prefix], look_ahead[name], name)
     words = look_ahead["mask"].numel()
@@ -175,8 +182,8 @@ def test_look_ahead_rows_equal_paced_rows_at_every_ring_position(hidden, rows):
     paced_rows = PACED_ELEMENTS // hidden + 37
     print(f"[schedules] ring H={hidden} rows={rows} (paced reference {paced_rows})", flush=True)
     case = make_case(paced_rows, hidden, torch.float16)
-    paced = run(case, paced_rows, torch.float32, 0.1, deterministic=True)
-    look_ahead = run(case, rows, torch.float32, 0.1, deterministic=True)
+    paced = run(case, paced_rows, torch.float32, 0.1, deterministic=True, walk=True)
+    look_ahead = run(case, rows, torch.float32, 0.1, deterministic=True, walk=True)
     for name in ROW_OUTPUTS:
         assert_same_bits(paced[name][:rows], look_ahead[name], name)
     words = look_ahead["mask"].numel()

@@ -122,7 +122,8 @@ def test_deterministic_partials(rows, hidden):
 
 
 @pytest.mark.parametrize("over", ["grad_normalized", "updated"])
-@pytest.mark.parametrize("rows,hidden", [(100, 768), (40, 2880)])
+@pytest.mark.parametrize("rows,hidden", [(100, 768), (40, 2880), (2047, 768), (4097, 768),
+                                         (6145, 768), (12291, 384), (4096, 832), (4096, 1024)])
 def test_gradients_written_over_their_inputs(rows, hidden, over):
     """grad_x in the memory of grad_normalized or `updated`: the same results
     as in memory of its own."""
@@ -147,8 +148,14 @@ def test_gradients_written_over_their_inputs(rows, hidden, over):
         results.append((grad_x, grad_branch, sums))
     assert torch.equal(results[0][0], results[1][0])
     assert torch.equal(results[0][1], results[1][1])
-    # Two fp32 orders of sums over at most 100 values of order one.
-    assert torch.allclose(results[0][2], results[1][2], rtol=1e-5, atol=1e-4)
+    separate, shared = results[0][2], results[1][2]
+    if rows <= 100:
+        # Two fp32 orders of sums over at most 100 values of order one.
+        assert torch.allclose(separate, shared, rtol=1e-5, atol=1e-4)
+    # Sums of n values of order one in two fp32 orders of at most 300 additions per
+    # term (rows of a wave or chunk, then blocks): 2^-24 * sqrt(300) = 1e-6 of the
+    # sums' norm, ten times that allowed.
+    assert ((separate - shared).norm(dim=1) <= 1e-5 * separate.norm(dim=1)).all()
 
 
 @pytest.mark.parametrize("rows,hidden", [(341, 768), (512, 1024), (64, 4096), (257, 2880), (5792, 128),

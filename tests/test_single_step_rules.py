@@ -178,3 +178,21 @@ def test_768_columns_with_32_bit_gradients_walk_from_7168_rows(ask):
                                            (704, F32, EVERYTHING), (832, F32, EVERYTHING)):
         assert ask([("backward", r, hidden, F16, grad_normalized, flags, 0, 1) for r in rows]) \
             == [[int(r * hidden <= 12 << 20)] for r in rows]
+
+
+def test_launches_named_after_walking_shapes_walk(ask):
+    """The GPU tests of the walking backward's shapes and schedules run in place or
+    deterministic: both take the walk at their sizes."""
+    import test_gpu_launch_shapes as shapes
+    import test_gpu_schedules as schedules
+
+    in_place = [(768, rows) for rows, _ in shapes.TWELVE_WAVE_CASES]
+    in_place += [(384, rows) for rows, _ in shapes.NINE_WAVE_CASES]
+    in_place += [(hidden, rows) for hidden, rows, _ in shapes.STAGGERED_WIDE_CASES]
+    in_place += schedules.RING_CASES
+    deterministic = [(hidden, rows) for hidden, rows, _ in shapes.STAGGERED_SHAPES]
+    queries = [("backward", rows, hidden, F16, F32, flags, 2, 1) for hidden, rows in in_place
+               for flags in (EVERYTHING, EVERYTHING | PARTIALS)]
+    queries += [("backward", rows, hidden, F16, F32, EVERYTHING | PARTIALS, 0, aligned)
+                for hidden, rows in deterministic for aligned in (0, 1)]
+    assert ask(queries) == [[0]] * len(queries)
