@@ -1508,23 +1508,30 @@ def kernel_name(kernel: str, workload: Workload) -> str:
 
 def launched_kernel(kernel: str, workload: Workload) -> str:
     """The kernel this workload launches: kernel_name()'s walking instance, or
-    the single-step kernel where the library's rules (rln_single.h
-    single_forward, single_backward, single_partials) take it."""
+    the single-step kernel where the library's rules for aligned tensors
+    (rln_single.h single_forward, single_backward) take it;
+    tests/test_single_step_rules.py holds this to them."""
     rows, hidden = workload.rows, workload.hidden
     elements = rows * hidden
     if kernel == "rln_forward_kernel":
-        if hidden > 4096 and not workload.dropout_p:
+        if hidden > 4096 and not workload.dropping:
             single = elements <= 1 << 17
         else:
-            single = rows <= 6144 and elements <= (1 << 21 if hidden <= 1280 else 1 << 20)
+            most_rows = 4096 if hidden == 128 and not workload.dropping else 6144
+            single = rows <= most_rows and elements <= (1 << 21 if hidden <= 1280 else 1 << 20)
+    elif workload.deterministic:
+        single = elements <= (384 << 10 if hidden == 128 else 256 << 10 if hidden == 192 else
+                              768 << 10 if hidden == 256 else 2 << 20 if hidden <= 768 else
+                              3 << 20 if hidden <= 2432 else 4 << 20 if hidden < 4096 else
+                              6 << 20 if hidden <= 6144 else 12 << 20)
     else:
-        most = (1 << 22 if hidden == 128 else 1 << 23 if hidden == 256 else
-                12 << 20 if hidden <= 1024 else 6 << 20 if hidden < 4096 else
-                1 << 23 if hidden <= 6144 else 1 << 24)
-        single = elements <= most and not (
-            workload.normalized == "f32" and rows >= 7168 and backward_twelve_waves(hidden, rows))
-        if workload.deterministic:
-            single = single and rows <= (4096 if hidden == 128 else 64 * 256)
+        wide = workload.branch == "f32" and workload.normalized == "f32"
+        single = elements <= (4 << 20 if hidden == 128 else 8 << 20 if hidden == 256 else
+                              7167 * 768 if hidden == 768 and workload.normalized == "f32" else
+                              12 << 20 if hidden <= 1024 else
+                              (4 << 20 if wide else 6 << 20) if hidden <= 3072 else
+                              3 << 20 if hidden < 4096 else 8 << 20 if hidden <= 6144 else
+                              16 << 20)
     if not single:
         return kernel_name(kernel, workload)
     return f"rln::{kernel.replace('rln_', 'rln_single_')} ({workload.branch}, {workload.normalized})"

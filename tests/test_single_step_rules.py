@@ -196,3 +196,34 @@ def test_launches_named_after_walking_shapes_walk(ask):
     queries += [("backward", rows, hidden, F16, F32, EVERYTHING | PARTIALS, 0, aligned)
                 for hidden, rows in deterministic for aligned in (0, 1)]
     assert ask(queries) == [[0]] * len(queries)
+
+
+def test_bench_names_the_kernel_the_rules_choose(ask):
+    """bench.py's roofline names the kernel a workload launches; its copy of the
+    rules agrees with the library's over sizes, dtypes and modes."""
+    import random
+    from dataclasses import replace
+
+    from test_bench_cli import _bench_module
+
+    bench = _bench_module()
+    code = {"f32": F32, "f16": F16, "bf16": BF16}
+    rng = random.Random(19)
+    workloads = [bench.C1, *bench.sweep_workloads()]
+    for hidden in HIDDEN:
+        for _ in range(24):
+            rows = max(1, round(2 ** rng.uniform(14, 25) / hidden))
+            workloads.append(replace(
+                bench.C1, rows=rows, hidden=hidden, branch=rng.choice(list(code)),
+                normalized=rng.choice(list(code)), dropout_p=rng.choice([0.0, 0.1]),
+                deterministic=rng.random() < 0.3, training=rng.random() < 0.8))
+    queries = []
+    for w in workloads:
+        flags = GRAD_UPDATED | GRAD_NORMALIZED | PARAMETERS | (PARTIALS if w.deterministic else 0)
+        queries.append(("forward", w.rows, w.hidden, w.dropping, 1))
+        queries.append(("backward", w.rows, w.hidden, code[w.branch], code[w.normalized], flags, 0, 1))
+    answers = ask(queries)
+    for w, forward, backward in zip(workloads, answers[::2], answers[1::2]):
+        named = [("single" in bench.launched_kernel(f"rln_{pass_}_kernel", w))
+                 for pass_ in ("forward", "backward")]
+        assert named == [bool(forward[0]), bool(backward[0])], w
